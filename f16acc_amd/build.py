@@ -36,6 +36,9 @@ ARCH = "gfx950"
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # MFMA results in vector registers also where a kernel may use accumulation
+    # registers (the quad kernel's chunk partials, which conversions read)
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wall", "-Wextra",
 ]
 HIP_FLAGS = COMMON_FLAGS + ["-fPIC", "-shared"]

@@ -49,6 +49,7 @@
 
 #include <atomic>
 #include <type_traits>
+#include <utility>
 
 #include "f16acc.h"
 
@@ -179,23 +180,35 @@ __device__ __forceinline__ void k_loop_generic(const Params& p, int64_t m0, int6
 // column-major inside a group, as the reference's _tile does,
 // kernel.py:26-29) so one XCD's tiles share A rows and B columns.
 // ---------------------------------------------------------------------------
-__host__ __device__ inline int64_t xcd_order(int64_t block, int64_t total) {
-  const int64_t x = block % kNumXcd, l = block / kNumXcd;
-  const int64_t q = total / kNumXcd, r = total % kNumXcd;
-  return x < r ? x * (q + 1) + l : r * (q + 1) + (x - r) * q + l;
+// The kernels compute it in 32 bits (T = uint32_t: a grid has at most 2^31 - 1
+// workgroups): in 64 bits the divisions were ~450 scalar instructions before a
+// workgroup's first copy, a microsecond of kernels that take seven.  A group's
+// width, kGroupM x tiles_n, is formed only where tiles_m > kGroupM, so it is
+// within 32 bits too.
+template <class T>
+__host__ __device__ inline T xcd_order(T block, T total) {
+  const T x = block % kNumXcd, l = block / kNumXcd;
+  const T q = total / kNumXcd, r = total % kNumXcd;
+  return x * q + (x < r ? x : r) + l;
 }
 
-__host__ __device__ inline void group_m(int64_t id, int64_t tiles_m, int64_t tiles_n, int64_t* tm, int64_t* tn) {
-  const int64_t width = kGroupM * tiles_n;
-  const int64_t first = (id / width) * kGroupM;
-  const int64_t gsz = tiles_m - first < kGroupM ? tiles_m - first : kGroupM;
-  *tm = first + (id % width) % gsz;
-  *tn = (id % width) / gsz;
+template <class T>
+__host__ __device__ inline void group_m(T id, T tiles_m, T tiles_n, int64_t* tm, int64_t* tn) {
+  T first = 0, gsz = tiles_m;
+  if (tiles_m > (T)kGroupM) {
+    const T width = kGroupM * tiles_n, group = id / width;
+    first = group * kGroupM;
+    gsz = tiles_m - first < (T)kGroupM ? tiles_m - first : kGroupM;
+    id -= group * width;
+  }
+  const T col = id / gsz;
+  *tm = first + (id - col * gsz);
+  *tn = col;
 }
 
 __host__ __device__ inline void block_tile(int64_t block, int64_t tiles_m, int64_t tiles_n, int64_t* tm,
                                            int64_t* tn) {
-  group_m(xcd_order(block, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
+  group_m<int64_t>(xcd_order<int64_t>(block, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
 }
 
 // LDS swizzles (see the header comment).  kc_swz spreads the 16 rows one
@@ -841,34 +854,18 @@ __device__ __forceinline__ void group_reduce(char LDS_AS* smem, int g, int ltid,
 // 0.9-1.4 % faster on 4096^3, 8192^3 and Qwen gate/up, level on the lm_head
 // shape.  (FP32 accumulation keeps k_loop_fast: there this form ran 2-6 %
 // slower.)
-
-//
-// entry (the persistent kernel's tile chaining): kIssueFirst, the loop
-// issues stage 0's copies itself; kFirstThenStores, they were issued before
-// exactly STORES more vector memory instructions of this wave (a tile's
-// output stores), so waiting until STORES remain outstanding has them
-// landed (vmcnt counts in issue order) while the stores drain; kFirstIssued,
-// issued before an unknown number of others: wait for everything.
-enum Entry { kIssueFirst = 0, kFirstThenStores = 1, kFirstIssued = 2 };
-
-template <class C, int STORES = 0>
+template <class C>
 __device__ __forceinline__ void k_loop_cross(const Params& p, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
                                              char LDS_AS* smem, FastLoader<C>& ld, int wave, int wm, int wn, int lane,
-                                             f32x4 (&acc)[C::FM][C::FN], int entry = kIssueFirst) {
+                                             f32x4 (&acc)[C::FM][C::FN]) {
   constexpr int T = C::FM * C::FN, kUnits = C::LA + C::LB;
   static_assert(kUnits <= T - C::FM, "copies must go out before the last column");
   static_assert(C::NS == 2 && C::KG == 1 && C::FM > 1, "two-stage ring, one K group");
   const int64_t nsteps = kend > kbeg ? (kend - kbeg + kStageK - 1) / kStageK : 0;
-  if (nsteps <= 0) {
-    if (entry != kIssueFirst) wait_vm0();  // a prefetched stage (zeros past K) must land before the LDS is reused
-    return;
-  }
+  if (nsteps <= 0) return;
   const int r16 = lane & 15, g = lane >> 4;
-  if (entry == kIssueFirst) ld.issue(p, m0, n0, kbeg, kend, smem, wave);
-  if (entry == kFirstThenStores)
-    wait_vm<STORES>();
-  else
-    wait_vm0();
+  ld.issue(p, m0, n0, kbeg, kend, smem, wave);
+  wait_vm0();
   __syncthreads();
   f16x8 af[C::FM][2], bc[2], bn[2];
   bc[0] = read_b<C>(smem + C::A_STAGE, wn, 0, 0, lane);
@@ -1467,119 +1464,611 @@ __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, 
 }
 
 // ---------------------------------------------------------------------------
-// Persistent chunked kernel for the 64x128-per-wave tiles (the table sends
-// 256x256 to it) on shapes of more than one round of tiles (the Qwen2.5-1.5B lm_head,
-// 2048 x 151936 x 1536: 18.6 rounds; 8192^3: 4).  One workgroup per CU
-// walks the tiles blockIdx.x, blockIdx.x + G, ... (G = gridDim.x, a multiple
-// of the 8 XCDs, so a workgroup keeps its XCD and round r runs the tiles a
-// one-tile-per-workgroup grid would run in its r-th round, in the same
-// block -> tile order).  At a tile's end the workgroup flags it (one
-// barrier), redoes it in FP32 if flagged (kernel.py:70-81), and then issues
-// the next tile's first-stage copies into ring slot 0 *before* staging and
-// storing this tile through the rest of the LDS: the next tile's first wait
-// covers those copies only (vmcnt counts in issue order, and exactly STORES
-// stores follow them in a wave with a whole sub-tile), so the stores drain
-// while the next tile's first stage is multiplied, and no workgroup launch,
-// prologue address setup or first-copy latency sits between tiles.
+// Chunked 256x256 kernel: chunk quads.
+//
+// The pair form above spends three MFMAs on two chunks.  Here four chunks of
+// a 16x16 block (a quad, 128 K) cost five: the four chunk MFMAs and one sparse
+// v_smfmac_f32_16x16x64_f16, which issues at the dense MFMA's rate and adds
+// four binary16 values per element into the FP32 sum against a constant 0/1
+// matrix (chunk_quad_selector): 2.5 MFMAs per chunk pair in place of 3.
+// What a quad needs at once, the fragments of 128 K, fits the registers only
+// with one wave per SIMD: four waves of 128x128 (512 registers each), the
+// FP32 sums in the 256 accumulation registers, and in the 256 vector registers
+// b's fragments of the whole quad (128), a's of the current and the next row
+// of blocks (32), two rounded quads and four partials in flight.  That also
+// reads a third less LDS per product than eight waves of 64x128.
+//
+// The bound is the chip's power: fed from registers alone, the loop's MFMAs
+// and conversions run at their full issue rate but at 1.69 GHz (3.04 us per
+// quad of a 256x256 tile, 97 us at 4096^3, where each MFMA's zero accumulator
+// and new operands toggle); the fragments, copies and barriers add the rest.
+// Measured per call against the pair form on eight waves, 4096^3 131 us
+// against 144 (w.t()), 8192^3 990 against 1078, 2048 x 8192 x 1536 55 against
+// 59.  Wider MFMAs (32x32x16, 14 % more power per product), copies spread
+// evenly over the quad (latency before the barrier that needs them: 1-3 %
+// slower) and streaming cache hints on the copies (4 % slower) were measured
+// and left out.
+//
+// LDS (160 KiB): b's quad (64 KiB) and a ring of three a halves (32 KiB each:
+// the rows of four of a wave's eight row blocks).  A quad walks its 64 blocks
+// row by row, b in registers, the next row's a fragments read one row ahead:
+//   Z  before block 4: every wave has read b(q) (in the last row of quad
+//      q - 1), so its LDS is free for b(q + 1): blocks 4-23 issue the copies of
+//      a(q + 1, half 0), whose slot was freed at Y of quad q - 1, and b(q + 1)
+//   X  before block 24: a(q, half 1) has landed (its reads start here) and
+//      a(q, half 0) is in registers: blocks 24-31 copy a(q + 1, half 1) into
+//      its slot
+//   Y  before block 56 (the last row): a(q + 1, half 0) and b(q + 1) have
+//      landed; the last row's blocks read them as each b column is done with.
+// The waits count outstanding copies (vmcnt is in issue order), so no copy
+// is waited for sooner than 32 blocks after its issue.
 // ---------------------------------------------------------------------------
-template <class C, bool OUT32>
-struct PersistentStore {
-  // the staging area: ring slot 1 onwards
-  static constexpr int AREA = C::RINGS - C::STAGE;
-  static constexpr int NW = C::WAVES_M * C::WAVES_N;
-  // fp16: the fewest column passes whose slices fit the area
-  static constexpr int P16 = passes(C::FN, (NW * C::WTM * C::WTN * 2 + AREA - 1) / AREA);
-  static constexpr int STORES16 = P16 * (C::WTM * (2 * C::FN / P16) / 64);
-  // fp32 (store_tile_staged32 with SMEM = AREA)
-  static constexpr int P32 = passes(C::FN, (NW * C::WTM * C::WTN * 4 + AREA - 1) / AREA);
-  static constexpr int STORES32 = P32 * (C::WTM * (C::WTN / P32 / 4) / 64);
-  static constexpr int STORES = OUT32 ? STORES32 : STORES16;
-  static_assert(STORES <= 63, "the stores must fit vmcnt");
-  static_assert(NW * C::WTM * (2 * C::WTN / P16) <= AREA, "fp16 staging slices must fit");
-  __device__ static __forceinline__ void store(const Params& p, char LDS_AS* area, int64_t m0, int64_t n0, int wave,
-                                               int wm, int wn, int lane, const f32x4 (&acc)[C::FM][C::FN]) {
-    if constexpr (OUT32)
-      store_tile_staged32<C, AREA>(p, m0, n0, wm, wn, lane, wave, area, acc);
+typedef f16 f16x16 __attribute__((ext_vector_type(16)));
+
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_seq(std::make_integer_sequence<int, N>{}, f);
+}
+
+template <int BM_, int BN_, int BL_>
+struct QuadCfg {
+  static constexpr int BM = BM_, BN = BN_, BL = BL_, WAVES_M = 2, WAVES_N = 2, T = 256;
+  static constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
+  static constexpr int QK = 4 * kChunk;                  // K of a quad
+  static constexpr int HALF = BM / 2 * QK * 2;           // bytes of an a half
+  static constexpr int B_AT = 3 * HALF, BQ = BN * QK * 2;  // b's place in the LDS, its bytes
+  static constexpr int LDS = B_AT + BQ;
+  static constexpr int UA = HALF / (T * 16), UBQ = BQ / (T * 16);  // 16-byte units a thread copies
+  static constexpr int UB = BN / 8;                      // NC: units per k-row
+  // the output is staged through the third a slot, 16 rows of a wave at a time
+  static constexpr int STAGE_AT = 2 * HALF, SLICE = HALF / 4;
+  static constexpr int stores(bool out32) { return WTM * WTN * (out32 ? 4 : 2) / 1024; }  // per wave
+  static_assert(LDS <= 160 * 1024 && 16 * WTN * 4 <= SLICE, "LDS of a CU");
+  static_assert(BL == kKC || T / UB == 8, "an NC unit's parity is bit 3 of its k-row");
+};
+
+// One copy of 16 bytes per lane to LDS, as lds_dma16, at lane offset base + step.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved: the asm sets it itself
+__device__ __forceinline__ void lds_dma16_step(const i32x4& srd, int lds, int base, int step) {
+  const int off = base + step;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, 0 offen lds"
+      :
+      : "s"(lds), "v"(off), "s"(srd)
+      : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// Copies of a quad (128 K) into the layouts of the 64-K stages above: a K-
+// contiguous operand's quad is two 64-K blocks one after the other, a
+// row-major b's 128 k-rows.  A unit's rows are a constant number of rows
+// below the lane's first: its offset is one addition, and rows past M (N;
+// k-rows past K) lie past the record count (FastLoader's rule).  A lane past
+// the quad's K range has the offset kOob, which stays past the record count
+// under every step (a tile's rows span fewer than 2^31 bytes, fast_layout).
+template <class C>
+struct QuadLoader {
+  i32x4 ra, rb;
+  int va[2], vb[2];  // lane offsets, by 64-K block (NC b: by unit parity)
+  int a_off, a_k, b_off[2];
+  int a_row, b_row;  // bytes per row of a, and of b (sbn) or per k-row (sbk)
+  int a_rec, b_rec;
+
+  __device__ __forceinline__ void init(const Params& p, int64_t m0, int64_t n0, int tid) {
+    const int row = tid >> 3, u = (tid & 7) ^ kc_swz(row);
+    a_row = __builtin_amdgcn_readfirstlane((int)(p.sam * 2));
+    a_off = row * a_row + u * 16;
+    a_k = 8 * u;
+    const int64_t ar = (p.M - m0) * p.sam * 2;
+    a_rec = __builtin_amdgcn_readfirstlane((int)(ar < kOob ? ar : kOob));
+    if (C::BL == kKC) {
+      b_row = __builtin_amdgcn_readfirstlane((int)(p.sbn * 2));
+      b_off[0] = row * b_row + u * 16;
+      b_off[1] = b_off[0] + 128;
+      const int64_t br = (p.N - n0) * p.sbn * 2;
+      b_rec = __builtin_amdgcn_readfirstlane((int)(br < kOob ? br : kOob));
+    } else {
+      b_row = __builtin_amdgcn_readfirstlane((int)(p.sbk * 2));
+      const int krow = tid / C::UB;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int ub = (tid % C::UB) ^ nc_swz(krow + 8 * s);
+        b_off[s] = n0 + 8 * ub < p.N ? krow * b_row + ub * 16 : kOob;
+      }
+      b_rec = 0;
+    }
+  }
+
+  // Resources and lane offsets of the quad at kbase, krem elements of K left.
+  __device__ __forceinline__ void quad(const Params& p, int64_t m0, int64_t n0, int64_t kbase, int krem) {
+    ra = make_srd(p.a + (m0 * p.sam + kbase));
+    ra[2] = a_rec;
+    va[0] = a_k < krem ? a_off : kOob;
+    va[1] = a_k + kStageK < krem ? a_off + 2 * kStageK : kOob;
+    if (C::BL == kKC) {
+      rb = make_srd(p.b + (n0 * p.sbn + kbase));
+      rb[2] = b_rec;
+      vb[0] = a_k < krem ? b_off[0] : kOob;  // (a lane copies the same k of both)
+      vb[1] = a_k + kStageK < krem ? b_off[1] : kOob;
+    } else {
+      rb = make_srd(p.b + (kbase * p.sbk + n0));
+      rb[2] = __builtin_amdgcn_readfirstlane((krem < C::QK ? krem : C::QK) * b_row);  // k-rows inside K
+      vb[0] = b_off[0];
+      vb[1] = b_off[1];
+    }
+  }
+
+  // Unit j of a's half h (rows [h WTM / 2, (h + 1) WTM / 2) of either wave row) to the slot at lds.
+  __device__ __forceinline__ void a_unit(int h, int j, int lds) const {
+    constexpr int PER = C::UA / 2, HW = C::WTM / 2;  // units and a wave row's rows in a 64-K block
+    const int row = 32 * (j % PER);
+    lds_dma16_step(ra, lds + j * C::T * 16, va[j / PER], (row / HW * C::WTM + h * HW + row % HW) * a_row);
+  }
+  __device__ __forceinline__ void b_unit(int j, int lds) const {
+    constexpr int PER = C::UBQ / 2;
+    if (C::BL == kKC)
+      lds_dma16_step(rb, lds + j * C::T * 16, vb[j / PER], 32 * (j % PER) * b_row);
     else
-      store_tile_staged<C, P16>(p, m0, n0, wm, wn, lane, wave, area, acc);
+      lds_dma16_step(rb, lds + j * C::T * 16, vb[j & 1], 8 * j * b_row);
+  }
+  // A tile's first quad: a half 0 to slot 0, b, a half 1 to slot 1 (lds: the LDS at this wave's units).
+  __device__ __forceinline__ void first(const Params& p, int64_t m0, int64_t n0, int lds) {
+    quad(p, m0, n0, 0, (int)p.K);
+#pragma unroll
+    for (int j = 0; j < C::UA; ++j) a_unit(0, j, lds);
+#pragma unroll
+    for (int j = 0; j < C::UBQ; ++j) b_unit(j, lds + C::B_AT);
+#pragma unroll
+    for (int j = 0; j < C::UA; ++j) a_unit(1, j, lds + C::HALF);
   }
 };
 
+// Fragment of a's row block i (its half's slot), chunk c of the quad.
+template <class C>
+__device__ __forceinline__ f16x8 quad_a(const char LDS_AS* slot, int wm, int i, int lane, int c) {
+  constexpr int HW = C::WTM / 2;
+  return read_kc<C>(slot + (c >> 1) * (C::HALF / 2), wm * HW + 16 * (i % (HW / 16)) + (lane & 15),
+                    4 * (c & 1) + (lane >> 4));
+}
+// Fragment of b's column block j, chunk c.
+template <class C>
+__device__ __forceinline__ f16x8 quad_b(const char LDS_AS* bs, int wn, int j, int lane, int c) {
+  if (C::BL == kKC)
+    return read_kc<C>(bs + (c >> 1) * (C::BQ / 2), wn * C::WTN + 16 * j + (lane & 15), 4 * (c & 1) + (lane >> 4));
+  return read_nc<C>(bs, wn * C::WTN + 16 * j, c, lane);
+}
+
+// Sparse selector of a chunk quad.  A chunk MFMA leaves lane 16q+m its
+// partials P[m][4q+r], r < 4; rounded, chunk c's four fill elements 4c..4c+3 of
+// an f16x16 X.  As the dense operand of v_smfmac_f32_16x16x64_f16, elements
+// 0-7 of lane 16q+m are K = 8q..8q+7 of column m and 8-15 K = 32+8q...: element
+// 4q+r of the output takes K = 8q+r, 8q+4+r, 32+8q+r, 32+8q+4+r, one value in
+// each of four groups of four.  The sparse operand's row i = 4q+r (lane 16l+i
+// holds K 16l..16l+15 as four groups of two stored values and their
+// positions) stores 1 at position r of groups 2(q%2), 2(q%2)+1 in lanes
+// l = q/2 and 2+q/2, and zeros elsewhere.
+__device__ __forceinline__ void chunk_quad_selector(int lane, f16x8& sel, int& idx) {
+  const int l = lane >> 4, q = (lane >> 2) & 3, r = lane & 3;
+  idx = 0;
+#pragma unroll
+  for (int grp = 0; grp < 4; ++grp) {
+    const bool on = (l & 1) == (q >> 1) && grp / 2 == (q & 1);
+    // stored values at positions (r, 3), or (0, 3) for r = 3
+    sel[2 * grp] = on && r < 3 ? (f16)1.0f : (f16)0.0f;
+    sel[2 * grp + 1] = on && r == 3 ? (f16)1.0f : (f16)0.0f;
+    idx |= ((r < 3 ? r : 0) | (3 << 2)) << (4 * grp);
+  }
+}
+
+// S += the quad's four rounded chunks.  The sum stays in accumulation
+// registers ("a"), which the compiler would otherwise not mix with partials in
+// vector registers.  Four MFMAs lie between the last conversion into x and
+// this read of it, and 60 blocks between two sums of one block.
+__device__ __forceinline__ void quad_sum(f32x4& s, const f16x8& sel, const f16x16& x, int idx) {
+  asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3" : "+a"(s) : "v"(sel), "v"(x), "v"(idx));
+}
+
+// A block's sum in vector registers.  Volatile asm: the compiler otherwise
+// moves all 64 blocks' reads ahead of the store's branches, and spills.
+__device__ __forceinline__ f32x4 quad_read(const f32x4& s) {
+  f32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float e;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(e) : "a"(s[r]));
+    v[r] = e;
+  }
+  return v;
+}
+
+// Chunk c of a quad: four partials rounded to binary16 (RNE, inf past 65504).
+__device__ __forceinline__ void quad_round(const f32x4& p, f16x16& x, int c) {
+  const f32x2 lo = {p[0], p[1]}, hi = {p[2], p[3]};
+  const f16x2 a = __builtin_convertvector(lo, f16x2), b = __builtin_convertvector(hi, f16x2);
+  x[4 * c] = a[0];
+  x[4 * c + 1] = a[1];
+  x[4 * c + 2] = b[0];
+  x[4 * c + 3] = b[1];
+}
+
+// What this wave has issued since its copies of a tile's first quad
+// (QuadLoader::first): nothing; exactly a whole sub-tile's stores, which may
+// stay outstanding while the copies are waited for (vmcnt counts in issue
+// order); or an unknown number of vector memory instructions.
+enum QuadSince { kNothing = 0, kStores = 1, kUnknown = 2 };
+
+// K loop of a tile whose first quad's copies have been issued.  Ends with a
+// barrier and the LDS free.
+template <class C, int STORES>
+__device__ __forceinline__ void k_loop_quad(const Params& p, int64_t m0, int64_t n0, char LDS_AS* smem,
+                                            QuadLoader<C>& ld, int lds, int wm, int wn, int lane, int since,
+                                            f32x4 (&acc)[C::FM][C::FN]) {
+  const int K = (int)p.K;
+  const char LDS_AS* bs = smem + C::B_AT;
+  constexpr int NB = C::FM * C::FN, HB = C::FM / 2;
+  constexpr int ZB = 4, XB = (HB - 1) * C::FN, YB = (C::FM - 1) * C::FN;
+  constexpr int U1 = C::UA + C::UBQ;
+  static_assert(C::FM % 2 == 0 && C::FN == 8 && U1 <= 2 * (XB - ZB) && XB + C::UA <= YB, "the schedule's places");
+  f16x8 bf[C::FN][4], af[2][4], sel;
+  f32x4 pr[4];   // partials of the last four chunk steps
+  f16x16 x[2];   // rounded quads of the last two blocks
+  int idx;
+  chunk_quad_selector(lane, sel, idx);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) pr[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  x[0] = x[1] = f16x16{};
+  if (since == kNothing)
+    wait_vm<C::UA>();  // a half 1 is waited for at X
+  else if (since == kStores)
+    wait_vm<STORES>();
+  else
+    wait_vm0();
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 4; ++c) af[0][c] = quad_a<C>(smem, wm, 0, lane, c);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) bf[j][c] = quad_b<C>(bs, wn, j, lane, c);
+  int s0 = 0, s1 = C::HALF, s2 = 2 * C::HALF;  // slots of a(q, 0), a(q, 1), a(q + 1, 0)
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (int kq = 0; kq < K; kq += C::QK) {
+    // past the K range every unit reads zeros into LDS no wave reads again
+    const int knext = kq + C::QK;
+    ld.quad(p, m0, n0, knext, K > knext ? K - knext : 0);
+    static_for<NB>([&](auto block) __attribute__((always_inline)) {
+      constexpr int b = block, i = b / C::FN, j = b % C::FN;
+      if constexpr (b == ZB) __syncthreads();
+      if constexpr (b == XB) {
+        wait_vm<U1>();
+        __syncthreads();
+      }
+      if constexpr (b == YB) {
+        wait_vm<C::UA>();
+        __syncthreads();
+      }
+      if constexpr (b >= ZB && b < XB) {
+        constexpr int u0 = (b - ZB) * U1 / (XB - ZB), u1 = (b - ZB + 1) * U1 / (XB - ZB);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int u = u0 + e;
+          if (u < u1 && u < C::UA) ld.a_unit(0, u, lds + s2);
+          if (u < u1 && u >= C::UA) ld.b_unit(u - C::UA, lds + C::B_AT);
+        }
+      }
+      if constexpr (b >= XB && b < XB + C::UA) ld.a_unit(1, b - XB, lds + s0);
+      constexpr int c0 = i == 0 ? j - ZB : j;  // the next row's a fragments (row 0: behind Z)
+      if constexpr (c0 >= 0 && c0 < 4) {
+        constexpr int ni = (i + 1) % C::FM;
+        af[(i + 1) & 1][c0] = quad_a<C>(smem + (ni == 0 ? s2 : ni < HB ? s0 : s1), wm, ni, lane, c0);
+      }
+      // Step s multiplies chunk c of block b, rounds step s - 3 (the fences
+      // keep the compiler from moving a conversion next to its MFMA) and, at
+      // a block's last chunk, sums the block before it.
+      static_for<4>([&](auto chunk) __attribute__((always_inline)) {
+        constexpr int c = chunk, s = 4 * b + c;
+        __builtin_amdgcn_sched_barrier(0);
+        pr[s % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j][c], af[i & 1][c], zero, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        quad_round(pr[(s + 1) % 4], x[(c == 3 ? b : b + 1) & 1], (c + 1) % 4);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (c == 3) {
+          constexpr int sb = (b + NB - 1) % NB;
+          quad_sum(acc[sb / C::FN][sb % C::FN], sel, x[(b + 1) & 1], idx);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      });
+      if constexpr (i == C::FM - 1) {  // b's column j is done with: the next quad's
+#pragma unroll
+        for (int c = 0; c < 4; ++c) bf[j][c] = quad_b<C>(bs, wn, j, lane, c);
+      }
+    });
+    const int t = s0;
+    s0 = s2;
+    s2 = s1;
+    s1 = t;
+  }
+  // the last block's chunks 1-3 and its sum
+#pragma unroll
+  for (int c = 1; c < 4; ++c) quad_round(pr[c], x[1], c);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 7");  // conversions, then an MFMA the compiler does not see
+  __builtin_amdgcn_sched_barrier(0);
+  quad_sum(acc[C::FM - 1][C::FN - 1], sel, x[1], idx);
+  __builtin_amdgcn_sched_barrier(0);
+  // (the same for the sums' next readers)
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  wait_vm0();       // the copies past the K range
+  __syncthreads();  // LDS free
+}
+
+// Whether a wave's sub-tile is stored whole: inside c, rows contiguous and 16-
+// byte aligned, offsets in 32 bits (C::stores() buffer stores).
 template <class C, bool OUT32>
-__global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) void gemm_persistent(Params p) {
-  static_assert(C::KG == 1 && C::NS == 2 && C::FM * C::FN >= 32, "the chunked 64x128-per-wave tiles");
-  using PS = PersistentStore<C, OUT32>;
-  __shared__ __attribute__((aligned(1024))) char smem_raw[C::RINGS];
-  __shared__ int flag_word[2];  // tile i raises word i & 1; the other is cleared meanwhile
+__device__ __forceinline__ bool quad_whole(const Params& p, int64_t m0, int64_t n0, int wm, int wn) {
+  return p.vec_store && p.M - m0 >= (wm + 1) * C::WTM && p.N - n0 >= (wn + 1) * C::WTN &&
+         C::WTM * p.scm * (OUT32 ? 4 : 2) < kOob;
+}
+
+// Store of a wave's 128x128 sums, staged like store_tile_staged but a row
+// block (16 rows) at a time through the wave's slice of the third a slot, so
+// that the next tile's first quad can land in the rest of the LDS meanwhile.
+// A wave's LDS operations run in order, so a block's reads follow its writes
+// without a wait; fp16 blocks alternate between the slice's halves, so that a
+// block is written while the one before it is read and stored.
+// Returns whether any sum is inf or NaN (kernel.py:70-71): 0 * s summed over
+// the lane's sums is zero exactly when all are finite.  fp16 outputs are tried
+// first, two a instruction (an inf or NaN sum is one in binary16 as well; so is
+// a finite sum past 65504, which the exact test then clears).
+template <class C, bool OUT32, bool BIASED>
+__device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, int64_t m0, int64_t n0, int wm, int wn,
+                                           int lane, const f32x4 (&acc)[C::FM][C::FN], const f16x8 (&bias)[4]) {
+  typedef f16 f16x4 __attribute__((ext_vector_type(4)));
+  constexpr int EL = OUT32 ? 4 : 8;         // elements of a 16-byte unit
+  constexpr int U = C::WTN / EL;            // units per row
+  constexpr int NU = 16 * U / 64;           // units a lane stores per row block
+  typedef std::conditional_t<OUT32, float, f16> Out;
+  typedef std::conditional_t<OUT32, f32x4, f16x8> Unit;
+  typedef std::conditional_t<OUT32, f32x4_a4, f16x8_a2> UnitAny;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int64_t col0 = n0 + wn * C::WTN, row0 = m0 + wm * C::WTM;
+  // whole sub-tiles: buffer stores, a lane offset per unit of a row block and
+  // a scalar offset per block, in place of a 64-bit address per store
+  const bool whole = quad_whole<C, OUT32>(p, m0, n0, wm, wn);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (Out*)p.c + row0 * p.scm + col0, (short)0, kOob, 0x00020000);
+  const int scm = __builtin_amdgcn_readfirstlane((int)p.scm) * (int)sizeof(Out);
+  float bad = 0.f;
+  f16x2 bad2 = {(f16)0.f, (f16)0.f};
+  auto write = [&](auto block) __attribute__((always_inline)) {
+    constexpr int i = block;
+    char LDS_AS* w = slice + (OUT32 ? 0 : (i & 1) * (C::SLICE / 2));
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) {
+      f32x4 v = quad_read(acc[i][j]);
+      if constexpr (OUT32 || BIASED) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bad = __builtin_fmaf(v[r], 0.f, bad);
+      }
+      if constexpr (BIASED) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float b = (float)bias[j / 2][4 * (j % 2) + r];
+          v[r] = OUT32 ? v[r] + b : (float)(f16)v[r] + b;  // with_bias
+        }
+      }
+      if constexpr (OUT32) {
+        *(f32x4 LDS_AS*)(w + r16 * (U * 16) + (((4 * j + g) ^ r16) << 4)) = v;
+      } else {
+        const f32x2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
+        const f16x2 hl = __builtin_convertvector(lo, f16x2), hh = __builtin_convertvector(hi, f16x2);
+        if constexpr (!BIASED) {
+          const f16x2 z = {(f16)0.f, (f16)0.f};
+          bad2 = __builtin_elementwise_fma(hl, z, bad2);
+          bad2 = __builtin_elementwise_fma(hh, z, bad2);
+        }
+        const f16x4 o = {hl[0], hl[1], hh[0], hh[1]};
+        *(f16x4 LDS_AS*)(w + r16 * (U * 16) + (((2 * j + (g >> 1)) ^ r16) << 4) + (g & 1) * 8) = o;
+      }
+    }
+    if constexpr (!OUT32 && !BIASED) {
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad2[0] == (f16)0.f && bad2[1] == (f16)0.f)) != 0, 0)) {
+        bad2 = f16x2{(f16)0.f, (f16)0.f};
+#pragma unroll
+        for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) bad = __builtin_fmaf(quad_read(acc[i][j])[r], 0.f, bad);
+      }
+    }
+    asm volatile("" : "+v"(bad));  // tested here, not at the end with every sum kept for it
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto unit = [&](int i, int it, int* row, int* col) __attribute__((always_inline)) {
+    const int id = it * 64 + lane, u = id % U;
+    *row = id / U;
+    *col = EL * u;
+    return *(const Unit LDS_AS*)(slice + (OUT32 ? 0 : (i & 1) * (C::SLICE / 2)) + *row * (U * 16) +
+                                 ((u ^ *row) << 4));
+  };
+  if (whole) {
+    Unit v[2][NU];
+    int off[NU];
+    static_for<C::FM + 1>([&](auto block) __attribute__((always_inline)) {
+      constexpr int i = block;
+      if constexpr (i < C::FM) write(block);
+      if constexpr (i < C::FM) {
+#pragma unroll
+        for (int it = 0; it < NU; ++it) {
+          int row, col;
+          v[i & 1][it] = unit(i, it, &row, &col);
+          if constexpr (i == 0) off[it] = row * scm + col * (int)sizeof(Out);
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+      if constexpr (i > 0) {
+#pragma unroll
+        for (int it = 0; it < NU; ++it)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v[(i - 1) & 1][it]), rs, off[it],
+                                                 16 * (i - 1) * scm, 0);
+      }
+    });
+  } else {
+    // the edges of c, and any strides: a loop of its own, whose masks stay
+    // out of the registers of the code above
+    const int64_t rows_in = p.M - row0, cols_in = p.N - col0;
+    const bool rows_ok = p.scn == 1 && ((uintptr_t)p.c & (sizeof(Out) - 1)) == 0;
+    static_for<C::FM>([&](auto block) __attribute__((always_inline)) {
+      constexpr int i = block;
+      write(block);
+#pragma unroll 1
+      for (int it = 0; it < NU; ++it) {
+        int row, col;
+        const Unit v = unit(i, it, &row, &col);
+        if (16 * i + row >= rows_in) continue;
+        Out* dst = (Out*)p.c + (row0 + 16 * i + row) * p.scm + (col0 + col) * p.scn;
+        if (rows_ok && col + EL <= cols_in) {
+          *(UnitAny*)dst = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < EL; ++e)
+            if (col + e < cols_in) dst[e * p.scn] = v[e];
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    });
+  }
+  return !(bad == 0.f);
+}
+
+// One tile per workgroup, or (a grid of one workgroup per CU on shapes of
+// more than one round: the Qwen2.5-1.5B lm_head, 8192^3) the tiles
+// blockIdx.x, blockIdx.x + G, ..., G a multiple of the 8 XCDs, in the block ->
+// tile order of a whole grid.  The next tile's first quad is copied before
+// this tile is stored, and the stores drain under its K loop.  An overflowing
+// tile (kernel.py:70-81) is listed for the redo launch (p.list) or redone
+// here, whole, with FP32 accumulation, as its four 128x128 quarters (C3): every
+// element sums the same products in the same order as the FP32 mode.
+template <class C, class C3, bool OUT32>
+__global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_quad(Params p) {
+  static_assert(C3::T == C::T && C3::BM * 2 == C::BM && C3::BN * 2 == C::BN && C3::RINGS <= C::LDS, "quarters");
+  __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
   char LDS_AS* smem = (char LDS_AS*)smem_raw;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
-  const int64_t tiles = p.tiles_m * p.tiles_n, G = gridDim.x;
-  int64_t t = blockIdx.x;
+  const int lds = __builtin_amdgcn_readfirstlane((int)(uint32_t)(size_t)smem + wave * 64 * 16);
+  const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n, tiles = tiles_m * tiles_n;
+  uint32_t t = blockIdx.x;
   if (t >= tiles) return;
-  if (tid == 0) flag_word[0] = flag_word[1] = 0;  // ordered before any raise by the K loop's barriers
   int64_t tm, tn;
-  group_m(xcd_order(t, tiles), p.tiles_m, p.tiles_n, &tm, &tn);
-  int entry = kIssueFirst;
-  for (int it = 0;; ++it) {
+  group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &tm, &tn);
+  bool issued = false;
+  int since = kNothing;
+  for (;;) {
     const int64_t m0 = tm * C::BM, n0 = tn * C::BN;
-    // The lane's index, opaque to the compiler once per tile: every
-    // lane-dependent address (LDS fragments, copies, staged stores) is then
-    // computed inside the tile loop instead of hoisted out of it and kept
-    // live across the K loop, where the registers are all taken (hoisted,
-    // they spilled around every tile).
+    // opaque once per tile: lane-dependent addresses are recomputed in the
+    // tile loop instead of kept (and spilled) across it
     int tid_t = tid;
     asm volatile("" : "+v"(tid_t));
-    const int lane_t = tid_t & 63;
-    FastLoader<C> ld;
-    ld.init(p, m0, n0, tid_t);
+    const int lane = tid_t & 63;
     f32x4 acc[C::FM][C::FN];
 #pragma unroll
     for (int i = 0; i < C::FM; ++i)
 #pragma unroll
       for (int j = 0; j < C::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    k_loop_cross<C, PS::STORES>(p, m0, n0, 0, p.K, smem, ld, wave, wm, wn, lane_t, acc, entry);
+    if (p.K > 0) {
+      QuadLoader<C> ld;
+      ld.init(p, m0, n0, tid_t);
+      if (!issued) ld.first(p, m0, n0, lds);
+      k_loop_quad<C, C::stores(OUT32) < 63 ? C::stores(OUT32) : 63>(p, m0, n0, smem, ld, lds, wm, wn, lane, since,
+                                                                     acc);
+    }
+    f16x8 bias[4] = {};  // this lane's columns: 16 j + 4 (lane / 16) + r
+    if (p.bias) {
+      const int64_t c0 = n0 + wn * C::WTN + 4 * (lane >> 4);
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int64_t col = c0 + 16 * (e / 4) + e % 4;
+        bias[e / 8][e % 8] = col < p.N ? p.bias[col] : (f16)0.f;
+      }
+      // waited for here: behind the next tile's copies a wait would include them
+      asm volatile("" : "+v"(bias[0]), "+v"(bias[1]), "+v"(bias[2]), "+v"(bias[3]));
+    }
+    t += gridDim.x;  // (no wrap: both are below 2^31)
+    const bool next = t < tiles && p.K > 0;
+    int64_t ntm = 0, ntn = 0;
+    if (t < tiles) group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &ntm, &ntn);
+    if (next) {
+      QuadLoader<C> nld;
+      nld.init(p, ntm * C::BM, ntn * C::BN, tid_t);
+      nld.first(p, ntm * C::BM, ntn * C::BN, lds);
+    }
+    issued = next;
+    since = !next ? kNothing : quad_whole<C, OUT32>(p, m0, n0, wm, wn) && !p.flags ? kStores : kUnknown;
+    char LDS_AS* slice = smem + C::STAGE_AT + wave * C::SLICE;
+    const bool bad = p.bias ? quad_store<C, OUT32, true>(p, slice, m0, n0, wm, wn, lane, acc, bias)
+                            : quad_store<C, OUT32, false>(p, slice, m0, n0, wm, wn, lane, acc, bias);
     if constexpr (kRedo) {
-      // tile flag: any element of the FP32 sum inf or NaN (kernel.py:70-71)
-      int LDS_AS* word = (int LDS_AS*)&flag_word[it & 1];
-      bool bad = false;
-#pragma unroll
-      for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) bad |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
-      if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane_t == 0) *word = 1;
+      // tile flag: one word at the start of the staging area
+      int LDS_AS* word = (int LDS_AS*)(smem + C::STAGE_AT);
+      if (tid_t == 0) *word = 0;  // wave 0's staging is done with it
+      __syncthreads();
+      if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *word = 1;
       __syncthreads();
       const int flag = *word;
-      // the other word's last reads were a tile ago; its next raise comes
-      // after the next tile's barriers
-      if (tid_t == 0) flag_word[(it + 1) & 1] = 0;
       if (p.flags && tid_t == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
-      if (__builtin_expect(flag, 0)) {
-        // redo the whole tile, all of K, with FP32 accumulation (kernel.py:75-81)
+      if (__builtin_expect(flag, 0) && !(kSplitRedo && p.defer_redo)) {
+        bool here = true;
+        __syncthreads();
+        if (p.list) {
+          // deferred: a list that is full (or not zeroed) leaves the redo here
+          if (tid_t == 0) {
+            const int at = atomicAdd(&p.list->alloc, 1);
+            const bool listed = at >= 0 && at < kRedoMax;
+            if (listed) {
+              store_agent(&p.list->items[at], (int)(tm * p.tiles_n + tn));
 #pragma unroll
-        for (int i = 0; i < C::FM; ++i)
+              for (int j = 0; j < kLines; ++j) atomicAdd(&p.list->line[j].word, 1ull);
+            }
+            *word = listed ? 2 : 1;
+          }
+          __syncthreads();
+          here = *word != 2;
+        }
+        if (here) {
+          wait_vm0();  // the next tile's copies have landed: the redo takes their place
+          __syncthreads();
+          for (int quarter = 0; quarter < 4; ++quarter) {
+            const int64_t qm = m0 + quarter / 2 * C3::BM, qn = n0 + quarter % 2 * C3::BN;
+            if (qm >= p.M || qn >= p.N) continue;
+            f32x4 sum[C3::FM][C3::FN];
 #pragma unroll
-          for (int j = 0; j < C::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        k_loop_fast<C, false>(p, m0, n0, 0, p.K, smem, ld, wave, wm, wn, lane_t, acc);
+            for (int i = 0; i < C3::FM; ++i)
+#pragma unroll
+              for (int j = 0; j < C3::FN; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            FastLoader<C3> fl;
+            fl.init(p, qm, qn, tid_t);
+            k_loop_fast<C3, false>(p, qm, qn, 0, p.K, smem, fl, wave, wm, wn, lane, sum);
+            store_any<C3, OUT32, C::LDS>(p, smem, qm, qn, wave, wm, wn, lane, sum);
+            __syncthreads();  // staging reads done before the next quarter's copies
+          }
+          issued = false;
+          since = kNothing;
+        }
       }
     }
-    t += G;
-    const bool next = t < tiles;
-    if (next) {
-      group_m(xcd_order(t, tiles), p.tiles_m, p.tiles_n, &tm, &tn);
-      FastLoader<C> nld;
-      nld.init(p, tm * C::BM, tn * C::BN, tid_t);
-      nld.issue(p, tm * C::BM, tn * C::BN, 0, p.K, smem, wave);  // into slot 0, free since the last barrier
-    }
-    PS::store(p, smem + C::STAGE, m0, n0, wave, wm, wn, lane_t, acc);
-    if (!next) return;
-    const int64_t rows_in = p.M - (m0 + wm * C::WTM), cols_in = p.N - (n0 + wn * C::WTN);
-    const bool whole = p.vec_store && rows_in >= C::WTM && cols_in >= C::WTN && !p.bias && !p.flags;
-    entry = whole ? kFirstThenStores : kFirstIssued;
-    __syncthreads();  // every wave's staging reads done: the next stage's copies may overwrite slot 1
+    if (t >= tiles) return;
+    tm = ntm;
+    tn = ntn;
   }
 }
 
@@ -1674,11 +2163,11 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) 
   // block -> (tile, K split): the XCD renumbering keeps a tile's splits together
   const int64_t tiles = p.tiles_m * p.tiles_n;
   const int nsplit = C::SPLITTABLE && p.mode == kPartial ? p.splits : 1;
-  const int64_t id = xcd_order(blockIdx.x, tiles * nsplit);
-  const int64_t tile = id / nsplit;
-  const int split = (int)(id % nsplit);
+  const uint32_t id = xcd_order<uint32_t>(blockIdx.x, (uint32_t)tiles * nsplit);
+  const uint32_t tile = nsplit > 1 ? id / (uint32_t)nsplit : id;
+  const int split = (int)(id - tile * nsplit);
   int64_t tm, tn;
-  group_m(tile, p.tiles_m, p.tiles_n, &tm, &tn);
+  group_m<uint32_t>(tile, (uint32_t)p.tiles_m, (uint32_t)p.tiles_n, &tm, &tn);
   if constexpr (kSplitRedo) {
     if (p.redo_only && !p.redo_only[(tm >> p.redo_sh) * p.redo_tn + (tn >> p.redo_sh)]) return;
   }
@@ -1709,7 +2198,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) 
   if (C::SPLITTABLE && p.mode == kPartial) {
     // buffer stores: one lane offset register and a scalar offset per
     // element, instead of a 64-bit address per store
-    float* mine = p.ws + (tile * p.splits + split) * (int64_t)(C::BM * C::BN);
+    float* mine = p.ws + ((int64_t)tile * p.splits + split) * (C::BM * C::BN);
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(mine, (short)0, C::BM * C::BN * (int)sizeof(float), 0x00020000);
 #pragma unroll
@@ -1738,14 +2227,14 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2))) void 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
-  const int64_t tile = xcd_order(blockIdx.x, p.tiles_m * p.tiles_n);
+  const uint32_t tile = xcd_order<uint32_t>(blockIdx.x, (uint32_t)(p.tiles_m * p.tiles_n));
   int64_t tm, tn;
-  group_m(tile, p.tiles_m, p.tiles_n, &tm, &tn);
+  group_m<uint32_t>(tile, (uint32_t)p.tiles_m, (uint32_t)p.tiles_n, &tm, &tn);
   if constexpr (kSplitRedo) {
     if (p.redo_only && !p.redo_only[(tm >> p.redo_sh) * p.redo_tn + (tn >> p.redo_sh)]) return;
   }
   if (CHUNKED && kRedo) tf.clear(tid);
-  const float* part = p.ws + tile * p.splits * (int64_t)(C::BM * C::BN);
+  const float* part = p.ws + (int64_t)tile * p.splits * (C::BM * C::BN);
   f32x4 acc[C::FM][C::FN];
 #pragma unroll
   for (int i = 0; i < C::FM; ++i)
@@ -2245,6 +2734,10 @@ inline Choice choose(int64_t M, int64_t N, int64_t K, int64_t sam, int64_t sak, 
   if (id == F16ACC_TILE_128x96_K2 && bl != kKC) id = F16ACC_TILE_128x128;
   if (id == F16ACC_TILE_64x32_K4 && bl != kKC) id = F16ACC_TILE_64x64;
   if (id == F16ACC_TILE_256x288 && bl != kKC) id = F16ACC_TILE_256x256;
+  // 256x256 copies 128 k-rows of a row-major b at a time (a quad), whose
+  // offsets must fit 32 bits as a stage's do.
+  if (id == F16ACC_TILE_256x256 && bl == kNC && (int64_t)4 * kChunk * sbk * 2 + 2 * kTiles[id].bn >= kOob)
+    id = F16ACC_TILE_128x128;
   if (bl >= 0) return Choice{id, F16ACC_FAMILY_FAST, bl};
   // Operands the copies cannot read: the tiles with registers to spare
   // stage them through registers (kReg); the others gather elements.  The
@@ -2261,20 +2754,25 @@ inline Choice choose(int64_t M, int64_t N, int64_t K, int64_t sam, int64_t sak, 
   return Choice{F16ACC_TILE_GENERIC, F16ACC_FAMILY_GENERIC, kKC};
 }
 
+// FP32 accumulation.
+template <class C, int LD>
+hipError_t launch_fp32(const Params& p, int out32, hipStream_t st) {
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * (p.mode == kPartial ? p.splits : 1))), block(C::T);
+  if (out32)
+    hipLaunchKernelGGL((gemm_kernel<C, LD, false, true>), grid, block, 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_kernel<C, LD, false, false>), grid, block, 0, st, p);
+  return hipGetLastError();
+}
+
 template <class C, int LD>
 hipError_t launch_cfg(const Params& p, int out32, int chunked, hipStream_t st) {
+  if (!chunked) return launch_fp32<C, LD>(p, out32, st);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * (p.mode == kPartial ? p.splits : 1))), block(C::T);
-  if (chunked) {
-    if (out32)
-      hipLaunchKernelGGL((gemm_kernel<C, LD, true, true>), grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_kernel<C, LD, true, false>), grid, block, 0, st, p);
-  } else {
-    if (out32)
-      hipLaunchKernelGGL((gemm_kernel<C, LD, false, true>), grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_kernel<C, LD, false, false>), grid, block, 0, st, p);
-  }
+  if (out32)
+    hipLaunchKernelGGL((gemm_kernel<C, LD, true, true>), grid, block, 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_kernel<C, LD, true, false>), grid, block, 0, st, p);
   return hipGetLastError();
 }
 
@@ -2284,12 +2782,18 @@ hipError_t launch_fast(const Params& p, int blayout, int out32, int chunked, hip
                         : launch_cfg<CF<kNC>, LD>(p, out32, chunked, st);
 }
 
-template <class C>
-hipError_t launch_persistent(const Params& p, int out32, int grid, hipStream_t st) {
+// Chunked 256x256: one workgroup per tile, or on shapes of more than one
+// round one per CU, each walking its tiles.
+template <int BL>
+hipError_t launch_quad(const Params& p, int out32, int cus, hipStream_t st) {
+  using C = QuadCfg<256, 256, BL>;
+  const int64_t tiles = p.tiles_m * p.tiles_n;
+  const bool persistent = kPersistent && tiles > cus && cus % kNumXcd == 0 && !p.defer_redo;
+  const dim3 grid((unsigned)(persistent ? cus : tiles)), block(C::T);
   if (out32)
-    hipLaunchKernelGGL((gemm_persistent<C, true>), dim3((unsigned)grid), dim3(C::T), 0, st, p);
+    hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true>), grid, block, 0, st, p);
   else
-    hipLaunchKernelGGL((gemm_persistent<C, false>), dim3((unsigned)grid), dim3(C::T), 0, st, p);
+    hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false>), grid, block, 0, st, p);
   return hipGetLastError();
 }
 
@@ -2514,7 +3018,12 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
       return ch.tile == F16ACC_TILE_64x64 ? (int)launch_cfg<Cfg5<kKC>, kReg>(q, out32, chunked, st)
                                           : (int)launch_fast<Cfg3, kReg>(q, ch.blayout, out32, chunked, st);
     switch (ch.tile) {
-      case 0: return (int)launch_fast<Cfg0>(q, ch.blayout, out32, chunked, st);
+      case 0:
+        if (chunked)
+          return ch.blayout == kKC ? (int)launch_quad<kKC>(q, out32, cu_count(), st)
+                                   : (int)launch_quad<kNC>(q, out32, cu_count(), st);
+        return ch.blayout == kKC ? (int)launch_fp32<Cfg0<kKC>, kDma>(q, out32, st)
+                                 : (int)launch_fp32<Cfg0<kNC>, kDma>(q, out32, st);
       case 1: return (int)launch_fast<Cfg1>(q, ch.blayout, out32, chunked, st);
       case 2: return (int)launch_fast<Cfg2>(q, ch.blayout, out32, chunked, st);
       case 3: return (int)launch_fast<Cfg3>(q, ch.blayout, out32, chunked, st);
@@ -2533,19 +3042,7 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
     if (!p.flags) p.flags = split_redo_flags();
     p.defer_redo = p.flags != nullptr;
   }
-  // Shapes of more than one round of 256x256 tiles, chunked, with
-  // contiguous output rows: one persistent workgroup per CU walks the tiles
-  // (gemm_persistent), chaining each tile's first copies ahead of the
-  // previous tile's store.  (256x288 keeps the grid: its persistent kernel
-  // spills a few registers per tile and ran 0.9 % slower on 8192 x 8960 x
-  // 1536.)
   const int cus = cu_count();
-  if (kPersistent && chunked && ch.family == F16ACC_FAMILY_FAST && p.mode == kWhole && !p.defer_redo && K > 0 &&
-      ch.tile == F16ACC_TILE_256x256 && scn == 1 && ((uintptr_t)c % 4) == 0 && p.tiles_m * p.tiles_n > cus &&
-      cus % kNumXcd == 0) {
-    return ch.blayout == kKC ? (int)launch_persistent<Cfg0<kKC>>(p, out32, cus, st)
-                             : (int)launch_persistent<Cfg0<kNC>>(p, out32, cus, st);
-  }
   int rc = launch(p);
   if (rc == 0 && p.defer_redo) return split_redo(p, redo_ws, ch.blayout, out32, st);
   if (rc == 0 && p.list) {
