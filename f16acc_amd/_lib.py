@@ -5,12 +5,16 @@ raises, and the package cannot be used.
 """
 
 import ctypes
+import importlib.util
 import os
 
-from .build import LIB
+import torch  # noqa: F401  (the native call path's module links against its libraries)
 
-if not os.path.exists(LIB):
-    raise ImportError(f"{LIB} is not built; run `python f16acc_amd/build.py` (needs hipcc for gfx950)")
+from .build import HOST, LIB
+
+for _f in (LIB, HOST):
+    if not os.path.exists(_f):
+        raise ImportError(f"{_f} is not built; run `python f16acc_amd/build.py` (needs hipcc for gfx950)")
 
 _dll = ctypes.CDLL(LIB)
 
@@ -89,3 +93,18 @@ if abi_version() != ABI_VERSION:
 def check(rc):
     if rc != 0:
         raise RuntimeError(strerror(rc).decode())
+
+
+def _load_host():
+    """The native call path (csrc/host.cpp)."""
+    spec = importlib.util.spec_from_file_location("f16acc_host", HOST)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+host = _load_host()
+
+
+def address(f):
+    return ctypes.cast(f, ctypes.c_void_p).value

@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 PKG = os.path.dirname(os.path.abspath(__file__))
@@ -29,6 +30,9 @@ LIB_SPLITREDO = os.path.join(OUT_DIR, "libf16acc_amd_splitredo.so")
 # of the persistent kernel (-DF16ACC_NO_PERSISTENT=1): only bench.py's
 # persistent A/B loads it.
 LIB_NOPERSIST = os.path.join(OUT_DIR, "libf16acc_amd_nopersist.so")
+# The native call path (csrc/host.cpp): a CPython module on torch's C++ headers.
+HOST_SRC = os.path.join(PKG, "csrc", "host.cpp")
+HOST = os.path.join(OUT_DIR, "f16acc_host.so")
 CHUNKRATE = os.path.join(OUT_DIR, "chunkrate")  # MFMA / chunk-epilogue microbenchmark
 ARCH = "gfx950"
 
@@ -51,12 +55,33 @@ def hipcc():
     raise FileNotFoundError("hipcc not found (set HIPCC or install ROCm under /opt/rocm)")
 
 
-def _start(flags, src, out):
-    """Start hipcc src -> a temporary file next to out."""
+def cxx():
+    cand = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cand:
+        raise FileNotFoundError("no host C++ compiler (set CXX or install g++)")
+    return cand
+
+
+def host_flags():
+    """Compile and link flags of the native call path for the installed torch
+    (its libraries are loaded by `import torch`, before this module)."""
+    import torch
+    from torch.utils import cpp_extension
+
+    flags = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unknown-pragmas", "-DUSE_ROCM=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for d in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]:
+        flags += ["-isystem", d]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return flags, [f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10"]
+
+
+def _start(flags, src, out, compiler=None, libs=()):
+    """Start hipcc (or `compiler`) src -> a temporary file next to out."""
     os.makedirs(OUT_DIR, exist_ok=True)
     fd, tmp = tempfile.mkstemp(suffix=".tmp", dir=OUT_DIR)
     os.close(fd)
-    cmd = [hipcc(), *flags, "-I", INCLUDE, src, "-o", tmp]
+    cmd = [compiler or hipcc(), *flags, "-I", INCLUDE, src, "-o", tmp, *libs]
     return cmd, tmp, out, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
 
 
@@ -66,7 +91,7 @@ def _finish(job, verbose):
     text, _ = proc.communicate()
     if proc.returncode != 0:
         os.unlink(tmp)
-        raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + text)
+        raise RuntimeError("compilation failed:\n" + " ".join(cmd) + "\n" + text)
     if verbose:
         noise = ("packed-fp32-ops", "warning generated", "warnings generated")
         msgs = [ln for ln in text.splitlines() if not any(n in ln for n in noise)]
@@ -78,12 +103,14 @@ def _finish(job, verbose):
 
 
 def build(verbose=False):
-    """Compile the library, its no-redo, split-redo and no-persistent twins
-    and the chunkrate microbenchmark (five hipcc processes at once)."""
+    """Compile the library, its no-redo, split-redo and no-persistent twins,
+    the chunkrate microbenchmark and the native call path (six compilers at
+    once)."""
+    flags, libs = host_flags()
     jobs = [_start(HIP_FLAGS, SRC, LIB), _start(HIP_FLAGS + ["-DF16ACC_NO_REDO=1"], SRC, LIB_NOREDO),
             _start(HIP_FLAGS + ["-DF16ACC_SPLIT_REDO=1"], SRC, LIB_SPLITREDO),
             _start(HIP_FLAGS + ["-DF16ACC_NO_PERSISTENT=1"], SRC, LIB_NOPERSIST),
-            _start(COMMON_FLAGS, CHUNKRATE_SRC, CHUNKRATE)]
+            _start(COMMON_FLAGS, CHUNKRATE_SRC, CHUNKRATE), _start(flags, HOST_SRC, HOST, cxx(), libs)]
     errors = []
     for job in jobs:
         try:

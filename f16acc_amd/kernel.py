@@ -22,6 +22,14 @@ _OUT = {torch.float16: _lib.OUT_F16, torch.float32: _lib.OUT_F32}
 # kernel (the copy's launch and traffic are not repaid).
 PACK_MIN_MACS = 1 << 24
 
+# The native call path (csrc/host.cpp) takes the calls whose operands go to the
+# kernels as they are and whose plan needs no workspace; it returns None for
+# every other call, which then takes the general path below.
+_host = _lib.host
+_compiling = torch.compiler.is_compiling  # a traced call takes the general path, as it did
+_host.setup(torch._C._cuda_getCurrentRawStream, PACK_MIN_MACS, *map(_lib.address, (
+    _lib.gemm, _lib.gemm_bias, _lib.workspace_size, _lib.tile_config, _lib.strerror)))
+
 # f16acc_tile_config's kernel families (F16ACC_FAMILY_* in include/f16acc.h)
 _FAMILIES = ("fast", "generic", "reg")
 
@@ -63,6 +71,15 @@ def mm(a, b, out_dtype=torch.float16, chunked=True):
                False -> plain FP32 accumulation
     Raises ValueError for bad shapes, dtypes or devices (kernel.py:87-90).
     """
+    if (out_dtype is torch.float16 or out_dtype is torch.float32) and not _compiling():
+        c = _host.mm(a, b, None, out_dtype is torch.float32, bool(chunked))
+        if c is not None:
+            return c
+    return _mm(a, b, out_dtype, chunked)
+
+
+def _mm(a, b, out_dtype, chunked):
+    """mm on the general path."""
     _validate(a, b, out_dtype)
     M, K = a.shape
     N = b.shape[1]
@@ -129,6 +146,15 @@ def mm_bias(a, b, bias, out_dtype=torch.float16, chunked=True):
     reference's unfused `y = mm(a, b); y += bias` (f16acc/patch.py:28-30) bit
     for bit: the FP32 sum is rounded to fp16, the bias added in FP32 and the
     sum rounded again, as torch's fp16 add does."""
+    if bias is not None and (out_dtype is torch.float16 or out_dtype is torch.float32) and not _compiling():
+        c = _host.mm(a, b, bias, out_dtype is torch.float32, bool(chunked))
+        if c is not None:
+            return c
+    return _mm_bias(a, b, bias, out_dtype, chunked)
+
+
+def _mm_bias(a, b, bias, out_dtype, chunked):
+    """mm_bias on the general path."""
     _validate(a, b, out_dtype)
     N = b.shape[1]
     if (bias.dim() != 1 or bias.shape[0] != N or bias.dtype != torch.float16 or not bias.is_cuda
