@@ -1676,6 +1676,12 @@ __device__ __forceinline__ void quad_sum(f32x4& s, const f16x8& sel, const f16x1
   asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3" : "+a"(s) : "v"(sel), "v"(x), "v"(idx));
 }
 
+// s += b a, one chunk, accumulating in FP32 (chunked = false), s in
+// accumulation registers as in quad_sum.
+__device__ __forceinline__ void quad_mac(f32x4& s, const f16x8& b, const f16x8& a) {
+  asm("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(s) : "v"(b), "v"(a));
+}
+
 // A block's sum in vector registers.  Volatile asm: the compiler otherwise
 // moves all 64 blocks' reads ahead of the store's branches, and spills.
 __device__ __forceinline__ f32x4 quad_read(const f32x4& s) {
@@ -1707,7 +1713,7 @@ enum QuadSince { kNothing = 0, kStores = 1, kUnknown = 2 };
 
 // K loop of a tile whose first quad's copies have been issued.  Ends with a
 // barrier and the LDS free.
-template <class C, int STORES>
+template <class C, bool CHUNKED, int STORES>
 __device__ __forceinline__ void k_loop_quad(const Params& p, int64_t m0, int64_t n0, char LDS_AS* smem,
                                             QuadLoader<C>& ld, int lds, int wm, int wn, int lane, int since,
                                             f32x4 (&acc)[C::FM][C::FN]) {
@@ -1770,25 +1776,38 @@ __device__ __forceinline__ void k_loop_quad(const Params& p, int64_t m0, int64_t
         constexpr int ni = (i + 1) % C::FM;
         af[(i + 1) & 1][c0] = quad_a<C>(smem + (ni == 0 ? s2 : ni < HB ? s0 : s1), wm, ni, lane, c0);
       }
-      // Step s multiplies chunk c of block b, rounds step s - 3 (the fences
-      // keep the compiler from moving a conversion next to its MFMA) and, at
-      // a block's last chunk, sums the block before it.
-      static_for<4>([&](auto chunk) __attribute__((always_inline)) {
-        constexpr int c = chunk, s = 4 * b + c;
-        __builtin_amdgcn_sched_barrier(0);
-        pr[s % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j][c], af[i & 1][c], zero, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        quad_round(pr[(s + 1) % 4], x[(c == 3 ? b : b + 1) & 1], (c + 1) % 4);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (c == 3) {
-          constexpr int sb = (b + NB - 1) % NB;
-          quad_sum(acc[sb / C::FN][sb % C::FN], sel, x[(b + 1) & 1], idx);
+      if constexpr (CHUNKED) {
+        // Step s multiplies chunk c of block b, rounds step s - 3 (the fences
+        // keep the compiler from moving a conversion next to its MFMA) and, at
+        // a block's last chunk, sums the block before it.
+        static_for<4>([&](auto chunk) __attribute__((always_inline)) {
+          constexpr int c = chunk, s = 4 * b + c;
           __builtin_amdgcn_sched_barrier(0);
-        }
-      });
-      if constexpr (i == C::FM - 1) {  // b's column j is done with: the next quad's
+          pr[s % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j][c], af[i & 1][c], zero, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          quad_round(pr[(s + 1) % 4], x[(c == 3 ? b : b + 1) & 1], (c + 1) % 4);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (c == 3) {
+            constexpr int sb = (b + NB - 1) % NB;
+            quad_sum(acc[sb / C::FN][sb % C::FN], sel, x[(b + 1) & 1], idx);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        });
+        if constexpr (i == C::FM - 1) {  // b's column j is done with: the next quad's
 #pragma unroll
-        for (int c = 0; c < 4; ++c) bf[j][c] = quad_b<C>(bs, wn, j, lane, c);
+          for (int c = 0; c < 4; ++c) bf[j][c] = quad_b<C>(bs, wn, j, lane, c);
+        }
+      } else {
+        // FP32 accumulation, two columns in turn, so that no MFMA waits for
+        // the one before it: chunks 0 and 1 of the pair at its first block, 2
+        // and 3 at its second.
+        static_for<4>([&](auto step) __attribute__((always_inline)) {
+          constexpr int c = 2 * (j & 1) + step / 2, col = (j & ~1) + step % 2;
+          __builtin_amdgcn_sched_barrier(0);
+          quad_mac(acc[i][col], bf[col][c], af[i & 1][c]);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (i == C::FM - 1) bf[col][c] = quad_b<C>(bs, wn, col, lane, c);
+        });
       }
     });
     const int t = s0;
@@ -1796,13 +1815,14 @@ __device__ __forceinline__ void k_loop_quad(const Params& p, int64_t m0, int64_t
     s2 = s1;
     s1 = t;
   }
-  // the last block's chunks 1-3 and its sum
+  if constexpr (CHUNKED) {  // the last block's chunks 1-3 and its sum
 #pragma unroll
-  for (int c = 1; c < 4; ++c) quad_round(pr[c], x[1], c);
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 7");  // conversions, then an MFMA the compiler does not see
-  __builtin_amdgcn_sched_barrier(0);
-  quad_sum(acc[C::FM - 1][C::FN - 1], sel, x[1], idx);
+    for (int c = 1; c < 4; ++c) quad_round(pr[c], x[1], c);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 7");  // conversions, then an MFMA the compiler does not see
+    __builtin_amdgcn_sched_barrier(0);
+    quad_sum(acc[C::FM - 1][C::FN - 1], sel, x[1], idx);
+  }
   __builtin_amdgcn_sched_barrier(0);
   // (the same for the sums' next readers)
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -1957,7 +1977,7 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
 // tile (kernel.py:70-81) is listed for the redo launch (p.list) or redone
 // here, whole, with FP32 accumulation, as its four 128x128 quarters (C3): every
 // element sums the same products in the same order as the FP32 mode.
-template <class C, class C3, bool OUT32>
+template <class C, class C3, bool CHUNKED, bool OUT32>
 __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_quad(Params p) {
   static_assert(C3::T == C::T && C3::BM * 2 == C::BM && C3::BN * 2 == C::BN && C3::RINGS <= C::LDS, "quarters");
   __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
@@ -1989,8 +2009,8 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
       QuadLoader<C> ld;
       ld.init(p, m0, n0, tid_t);
       if (!issued) ld.first(p, m0, n0, lds);
-      k_loop_quad<C, C::stores(OUT32) < 63 ? C::stores(OUT32) : 63>(p, m0, n0, smem, ld, lds, wm, wn, lane, since,
-                                                                     acc);
+      constexpr int kStores = C::stores(OUT32) < 63 ? C::stores(OUT32) : 63;
+      k_loop_quad<C, CHUNKED, kStores>(p, m0, n0, smem, ld, lds, wm, wn, lane, since, acc);
     }
     f16x8 bias[4] = {};  // this lane's columns: 16 j + 4 (lane / 16) + r
     if (p.bias) {
@@ -2015,9 +2035,9 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
     issued = next;
     since = !next ? kNothing : quad_whole<C, OUT32>(p, m0, n0, wm, wn) && !p.flags ? kStores : kUnknown;
     char LDS_AS* slice = smem + C::STAGE_AT + wave * C::SLICE;
-    const bool bad = p.bias ? quad_store<C, OUT32, true>(p, slice, m0, n0, wm, wn, lane, acc, bias)
+    [[maybe_unused]] const bool bad = p.bias ? quad_store<C, OUT32, true>(p, slice, m0, n0, wm, wn, lane, acc, bias)
                             : quad_store<C, OUT32, false>(p, slice, m0, n0, wm, wn, lane, acc, bias);
-    if constexpr (kRedo) {
+    if constexpr (CHUNKED && kRedo) {
       // tile flag: one word at the start of the staging area
       int LDS_AS* word = (int LDS_AS*)(smem + C::STAGE_AT);
       if (tid_t == 0) *word = 0;  // wave 0's staging is done with it
@@ -2307,7 +2327,6 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 //   6   128x96   2 x 4  64x48      (2 + 3) x 28 KiB  1   (two K groups, split phases)
 //   7   64x32    4 x 2  32x32      2 x (2 + 3) x 12 KiB  1   (four K groups, split phases)
 //   8   256x288  8      64x144     2 x 68 KiB    1   (K-contiguous b)
-template <int BL> using Cfg0 = Cfg<256, 256, 4, 2, 2, BL>;
 template <int BL> using Cfg1 = Cfg<256, 128, 4, 2, 3, BL>;
 template <int BL> using Cfg2 = Cfg<128, 256, 2, 4, 3, BL>;
 template <int BL> using Cfg3 = Cfg<128, 128, 2, 2, 2, BL>;
@@ -2754,25 +2773,20 @@ inline Choice choose(int64_t M, int64_t N, int64_t K, int64_t sam, int64_t sak, 
   return Choice{F16ACC_TILE_GENERIC, F16ACC_FAMILY_GENERIC, kKC};
 }
 
-// FP32 accumulation.
-template <class C, int LD>
-hipError_t launch_fp32(const Params& p, int out32, hipStream_t st) {
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * (p.mode == kPartial ? p.splits : 1))), block(C::T);
-  if (out32)
-    hipLaunchKernelGGL((gemm_kernel<C, LD, false, true>), grid, block, 0, st, p);
-  else
-    hipLaunchKernelGGL((gemm_kernel<C, LD, false, false>), grid, block, 0, st, p);
-  return hipGetLastError();
-}
-
 template <class C, int LD>
 hipError_t launch_cfg(const Params& p, int out32, int chunked, hipStream_t st) {
-  if (!chunked) return launch_fp32<C, LD>(p, out32, st);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * (p.mode == kPartial ? p.splits : 1))), block(C::T);
-  if (out32)
-    hipLaunchKernelGGL((gemm_kernel<C, LD, true, true>), grid, block, 0, st, p);
-  else
-    hipLaunchKernelGGL((gemm_kernel<C, LD, true, false>), grid, block, 0, st, p);
+  if (chunked) {
+    if (out32)
+      hipLaunchKernelGGL((gemm_kernel<C, LD, true, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_kernel<C, LD, true, false>), grid, block, 0, st, p);
+  } else {
+    if (out32)
+      hipLaunchKernelGGL((gemm_kernel<C, LD, false, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_kernel<C, LD, false, false>), grid, block, 0, st, p);
+  }
   return hipGetLastError();
 }
 
@@ -2782,18 +2796,25 @@ hipError_t launch_fast(const Params& p, int blayout, int out32, int chunked, hip
                         : launch_cfg<CF<kNC>, LD>(p, out32, chunked, st);
 }
 
-// Chunked 256x256: one workgroup per tile, or on shapes of more than one
-// round one per CU, each walking its tiles.
+// 256x256: one workgroup per tile, or on shapes of more than one round one
+// per CU, each walking its tiles.
 template <int BL>
-hipError_t launch_quad(const Params& p, int out32, int cus, hipStream_t st) {
+hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStream_t st) {
   using C = QuadCfg<256, 256, BL>;
   const int64_t tiles = p.tiles_m * p.tiles_n;
   const bool persistent = kPersistent && tiles > cus && cus % kNumXcd == 0 && !p.defer_redo;
   const dim3 grid((unsigned)(persistent ? cus : tiles)), block(C::T);
-  if (out32)
-    hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true>), grid, block, 0, st, p);
-  else
-    hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false>), grid, block, 0, st, p);
+  if (chunked) {
+    if (out32)
+      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true, false>), grid, block, 0, st, p);
+  } else {
+    if (out32)
+      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false, false>), grid, block, 0, st, p);
+  }
   return hipGetLastError();
 }
 
@@ -3019,11 +3040,8 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
                                           : (int)launch_fast<Cfg3, kReg>(q, ch.blayout, out32, chunked, st);
     switch (ch.tile) {
       case 0:
-        if (chunked)
-          return ch.blayout == kKC ? (int)launch_quad<kKC>(q, out32, cu_count(), st)
-                                   : (int)launch_quad<kNC>(q, out32, cu_count(), st);
-        return ch.blayout == kKC ? (int)launch_fp32<Cfg0<kKC>, kDma>(q, out32, st)
-                                 : (int)launch_fp32<Cfg0<kNC>, kDma>(q, out32, st);
+        return ch.blayout == kKC ? (int)launch_quad<kKC>(q, out32, chunked, cu_count(), st)
+                                 : (int)launch_quad<kNC>(q, out32, chunked, cu_count(), st);
       case 1: return (int)launch_fast<Cfg1>(q, ch.blayout, out32, chunked, st);
       case 2: return (int)launch_fast<Cfg2>(q, ch.blayout, out32, chunked, st);
       case 3: return (int)launch_fast<Cfg3>(q, ch.blayout, out32, chunked, st);
