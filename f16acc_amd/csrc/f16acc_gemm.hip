@@ -1142,10 +1142,51 @@ __device__ __forceinline__ void k_loop_generic(const Params& p, int64_t m0, int6
 // sum is rounded to binary16 first, the bias is added in FP32 and the result
 // rounded again.  An FP32 output adds the bias to the FP32 sum directly.
 template <bool OUT32>
-__device__ __forceinline__ float with_bias(float v, const f16* bias, int64_t col) {
-  if (!bias) return v;
-  const float b = (float)bias[col];
-  return OUT32 ? v + b : (float)(f16)v + b;
+__device__ __forceinline__ float with_bias(float v, f16 bias) {
+  return OUT32 ? v + (float)bias : (float)(f16)v + (float)bias;
+}
+
+// The bias of a lane's columns: 16 j + 4 (lane / 16) + r of its wave's sub-tile,
+// every load in flight at once (a load per element behind its own bounds test,
+// in the store, cost 4 us a call on 2048 x 1536 x 1536).  Columns past N take the
+// last one's; they are not stored.
+typedef f16 f16x4 __attribute__((ext_vector_type(4)));
+typedef f16x4 __attribute__((aligned(2))) f16x4_a2;
+template <class C>
+struct Bias {
+  f16x4 v[C::FN];
+  __device__ __forceinline__ Bias(const Params& p, int64_t n0, int wn, int lane) {
+    const int64_t col0 = n0 + wn * C::WTN;
+    const int g4 = 4 * (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) v[j] = f16x4{};
+    if (!p.bias) return;
+    if (col0 + C::WTN <= p.N) {  // wave-uniform
+#pragma unroll
+      for (int j = 0; j < C::FN; ++j) v[j] = *(const f16x4_a2*)(p.bias + col0 + 16 * j + g4);
+    } else {
+#pragma unroll
+      for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t col = col0 + 16 * j + g4 + r;
+          v[j][r] = p.bias[col < p.N ? col : p.N - 1];
+        }
+    }
+  }
+};
+
+// In place of a bias loaded early: it is loaded where it is stored with.
+struct LateBias {
+  __device__ __forceinline__ LateBias(const Params&, int64_t, int, int) {}
+};
+template <class C>
+__device__ __forceinline__ Bias<C> bias_at_store(const LateBias&, const Params& p, int64_t n0, int wn, int lane) {
+  return Bias<C>(p, n0, wn, lane);
+}
+template <class C>
+__device__ __forceinline__ const Bias<C>& bias_at_store(const Bias<C>& early, const Params&, int64_t, int, int) {
+  return early;
 }
 
 // Staging position of 16-byte unit u of a staged row: XOR-swizzled by row so
@@ -1176,8 +1217,8 @@ __device__ __forceinline__ int stg_swz(int u, int row) {
 // sub-tile is whole issues exactly P * WTM * (2 FN / P) / 64 stores.
 template <class C, int P = 1>
 __device__ __forceinline__ void store_tile_staged(const Params& p, int64_t m0, int64_t n0, int wm, int wn, int lane,
-                                                  int wave, char LDS_AS* smem, const f32x4 (&acc)[C::FM][C::FN]) {
-  typedef f16 f16x4 __attribute__((ext_vector_type(4)));
+                                                  int wave, char LDS_AS* smem, const f32x4 (&acc)[C::FM][C::FN],
+                                                  const Bias<C>& bias) {
   static_assert(C::FN % P == 0, "passes split the column blocks evenly");
   constexpr int FNP = C::FN / P;  // column blocks per pass
   constexpr int U = 2 * FNP;      // 16-byte units per staged row
@@ -1199,10 +1240,7 @@ __device__ __forceinline__ void store_tile_staged(const Params& p, int64_t m0, i
         f32x4 v = acc[i][j];
         if (p.bias) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int64_t col = col0 + 16 * j + 4 * g + r;
-            if (col < p.N) v[r] = with_bias<false>(v[r], p.bias, col);
-          }
+          for (int r = 0; r < 4; ++r) v[r] = with_bias<false>(v[r], bias.v[j][r]);
         }
         const f32x2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
         const f16x2 hl = __builtin_convertvector(lo, f16x2), hh = __builtin_convertvector(hi, f16x2);
@@ -1253,7 +1291,7 @@ constexpr int passes(int fn, int least) {
 template <class C, int SMEM>
 __device__ __forceinline__ void store_tile_staged32(const Params& p, int64_t m0, int64_t n0, int wm, int wn,
                                                     int lane, int wave, char LDS_AS* smem,
-                                                    const f32x4 (&acc)[C::FM][C::FN]) {
+                                                    const f32x4 (&acc)[C::FM][C::FN], const Bias<C>& bias) {
   constexpr int NW = C::WAVES_M * C::WAVES_N;
   constexpr int P = passes(C::FN, (NW * C::WTM * C::WTN * 4 + SMEM - 1) / SMEM);
   constexpr int PW = C::WTN / P;  // columns per pass
@@ -1277,10 +1315,7 @@ __device__ __forceinline__ void store_tile_staged32(const Params& p, int64_t m0,
         f32x4 v = acc[i][j];
         if (p.bias) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int64_t col = col0 + 16 * j + 4 * g + r;
-            if (col < p.N) v[r] = with_bias<true>(v[r], p.bias, col);
-          }
+          for (int r = 0; r < 4; ++r) v[r] = with_bias<true>(v[r], bias.v[j][r]);
         }
         *(f32x4 LDS_AS*)(w + row * ROW + (stg_swz<U>(u, row) << 4)) = v;
       }
@@ -1309,7 +1344,7 @@ __device__ __forceinline__ void store_tile_staged32(const Params& p, int64_t m0,
 
 template <class C, bool OUT32>
 __device__ __forceinline__ void store_tile(const Params& p, int64_t m0, int64_t n0, int wm, int wn, int lane,
-                                           const f32x4 (&acc)[C::FM][C::FN]) {
+                                           const f32x4 (&acc)[C::FM][C::FN], const Bias<C>& bias) {
   const int r16 = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int i = 0; i < C::FM; ++i) {
@@ -1319,17 +1354,16 @@ __device__ __forceinline__ void store_tile(const Params& p, int64_t m0, int64_t 
     for (int j = 0; j < C::FN; ++j) {
       const int64_t col = n0 + wn * C::WTN + 16 * j + 4 * g;
       f32x4 v = acc[i][j];
-      if (p.vec_store && col + 3 < p.N) {
-        if (p.bias) {
+      if (p.bias) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = with_bias<OUT32>(v[r], p.bias, col + r);
-        }
+        for (int r = 0; r < 4; ++r) v[r] = with_bias<OUT32>(v[r], bias.v[j][r]);
+      }
+      if (p.vec_store && col + 3 < p.N) {
         if (OUT32) {
           *(f32x4*)((float*)p.c + row * p.scm + col) = v;
         } else {
           const f32x2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
           const f16x2 hl = __builtin_convertvector(lo, f16x2), hh = __builtin_convertvector(hi, f16x2);
-          typedef f16 f16x4 __attribute__((ext_vector_type(4)));
           const f16x4 o = {hl[0], hl[1], hh[0], hh[1]};
           *(f16x4*)((f16*)p.c + row * p.scm + col) = o;
         }
@@ -1338,11 +1372,10 @@ __device__ __forceinline__ void store_tile(const Params& p, int64_t m0, int64_t 
         for (int r = 0; r < 4; ++r) {
           if (col + r >= p.N) break;
           const int64_t off = row * p.scm + (col + r) * p.scn;
-          const float o = with_bias<OUT32>(v[r], p.bias, col + r);
           if (OUT32)
-            ((float*)p.c)[off] = o;
+            ((float*)p.c)[off] = v[r];
           else
-            ((f16*)p.c)[off] = (f16)o;
+            ((f16*)p.c)[off] = (f16)v[r];
         }
       }
     }
@@ -1372,13 +1405,13 @@ struct TileFlag {
 // (needs the LDS free: every wave's reads of the last K stage done).
 template <class C, bool OUT32, int SMEM>
 __device__ __forceinline__ void store_any(const Params& p, char LDS_AS* smem, int64_t m0, int64_t n0, int wave, int wm,
-                                          int wn, int lane, const f32x4 (&acc)[C::FM][C::FN]) {
+                                          int wn, int lane, const f32x4 (&acc)[C::FM][C::FN], const Bias<C>& bias) {
   if (!OUT32 && C::BM * C::BN * 2 <= SMEM && p.scn == 1)
-    store_tile_staged<C>(p, m0, n0, wm, wn, lane, wave, smem, acc);
+    store_tile_staged<C>(p, m0, n0, wm, wn, lane, wave, smem, acc, bias);
   else if (OUT32 && p.scn == 1 && ((uintptr_t)p.c & 3) == 0)
-    store_tile_staged32<C, SMEM>(p, m0, n0, wm, wn, lane, wave, smem, acc);
+    store_tile_staged32<C, SMEM>(p, m0, n0, wm, wn, lane, wave, smem, acc, bias);
   else
-    store_tile<C, OUT32>(p, m0, n0, wm, wn, lane, acc);
+    store_tile<C, OUT32>(p, m0, n0, wm, wn, lane, acc, bias);
 }
 
 // Flag, redo and store of a finished FP32 tile sum (shared by the whole-K
@@ -1395,10 +1428,11 @@ __device__ __forceinline__ void store_any(const Params& p, char LDS_AS* smem, in
 // barriers, and a redo runs as the main pass did, each group over its own K
 // range (in FP32), then the same reduction.  g is the thread's K group, lw
 // its wave inside the group, ltid its thread inside the group.
-template <class C, int LD, bool CHUNKED, bool OUT32, int SMEM>
+template <class C, int LD, bool CHUNKED, bool OUT32, int SMEM, class B>
 __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, FastLoader<C>& ld, const RegLoader<C>& rl,
                                             const TileFlag& tf, int64_t tm, int64_t tn, int tid, int g, int ltid,
-                                            int lw, int wm, int wn, int lane, f32x4 (&acc)[C::FM][C::FN]) {
+                                            int lw, int wm, int wn, int lane, f32x4 (&acc)[C::FM][C::FN],
+                                            const B& bias) {
   const int64_t m0 = tm * C::BM, n0 = tn * C::BN;
   if constexpr (CHUNKED && kRedo && C::KG > 1) {
     // the flag word was raised before group_reduce's last barrier: no store
@@ -1423,7 +1457,7 @@ __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, 
         for (int j = 0; j < C::FN; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) bad |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
-      store_any<C, OUT32, SMEM>(p, smem, m0, n0, lw, wm, wn, lane, acc);
+      store_any<C, OUT32, SMEM>(p, smem, m0, n0, lw, wm, wn, lane, acc, bias_at_store<C>(bias, p, n0, wn, lane));
     }
     // the flag's barrier also retires every wave's reads of its LDS staging
     // slice before a redo's copies overwrite the LDS
@@ -1460,7 +1494,8 @@ __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, 
     else
       k_loop_generic<C, false>(p, m0, n0, smem, tid, wm, wn, lane, acc);
   }
-  if (g == 0) store_any<C, OUT32, SMEM>(p, smem, m0, n0, lw, wm, wn, lane, acc);
+  if (g == 0)
+    store_any<C, OUT32, SMEM>(p, smem, m0, n0, lw, wm, wn, lane, acc, bias_at_store<C>(bias, p, n0, wn, lane));
 }
 
 // ---------------------------------------------------------------------------
@@ -2078,7 +2113,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
             FastLoader<C3> fl;
             fl.init(p, qm, qn, tid_t);
             k_loop_fast<C3, false>(p, qm, qn, 0, p.K, smem, fl, wave, wm, wn, lane, sum);
-            store_any<C3, OUT32, C::LDS>(p, smem, qm, qn, wave, wm, wn, lane, sum);
+            store_any<C3, OUT32, C::LDS>(p, smem, qm, qn, wave, wm, wn, lane, sum, Bias<C3>(p, qn, wn, lane));
             __syncthreads();  // staging reads done before the next quarter's copies
           }
           issued = false;
@@ -2142,7 +2177,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) 
     FastLoader<C> ld;
     ld.init(p, m0, n0, tid);
     k_loop_fast<C, false>(p, m0, n0, 0, p.K, smem, ld, wave, wm, wn, lane, acc);
-    store_any<C, OUT32, kSmem>(p, smem, m0, n0, wave, wm, wn, lane, acc);
+    store_any<C, OUT32, kSmem>(p, smem, m0, n0, wave, wm, wn, lane, acc, Bias<C>(p, n0, wn, lane));
     __syncthreads();  // staging reads done before the next quarter's copies
   }
 }
@@ -2204,6 +2239,9 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) 
 
   FastLoader<C> ld;
   RegLoader<C> rl;
+  // the K-group tiles' short calls load their bias before the K loop (4
+  // registers), the others, whose registers are full, after it
+  std::conditional_t<(C::KG > 1), Bias<C>, LateBias> bias(p, n0, wn, lane);
   if constexpr (LD == kDma) {
     ld.init(p, m0, n0, ltid);
     k_groups_fast<C, CHUNKED>(p, m0, n0, kbeg, kend, smem, ld, g, ltid, lw, wm, wn, lane, acc,
@@ -2229,7 +2267,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) 
                                                part_offset<C>(i, j, 0) * 4, 0);
     return;
   }
-  finish_tile<C, LD, CHUNKED, OUT32, kSmem>(p, smem, ld, rl, tf, tm, tn, tid, g, ltid, lw, wm, wn, lane, acc);
+  finish_tile<C, LD, CHUNKED, OUT32, kSmem>(p, smem, ld, rl, tf, tm, tn, tid, g, ltid, lw, wm, wn, lane, acc, bias);
 }
 
 // Split-K finishing kernel (kFinish): one workgroup per tile adds the FP32
@@ -2254,6 +2292,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2))) void 
     if (p.redo_only && !p.redo_only[(tm >> p.redo_sh) * p.redo_tn + (tn >> p.redo_sh)]) return;
   }
   if (CHUNKED && kRedo) tf.clear(tid);
+  const Bias<C> bias(p, tn * C::BN, wn, lane);  // in flight with the partials
   const float* part = p.ws + (int64_t)tile * p.splits * (C::BM * C::BN);
   f32x4 acc[C::FM][C::FN];
 #pragma unroll
@@ -2271,7 +2310,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(2))) void 
   RegLoader<C> unused_rl;
   static_assert(C::KG == 1, "split-K tiles have one K group");
   finish_tile<C, kGather, CHUNKED, OUT32, kSmem>(p, smem, unused, unused_rl, tf, tm, tn, tid, 0, tid, wave, wm, wn,
-                                                 lane, acc);
+                                                 lane, acc, bias);
 }
 
 // ---------------------------------------------------------------------------
