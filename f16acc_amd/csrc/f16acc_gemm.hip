@@ -2127,6 +2127,305 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
   }
 }
 
+// ---------------------------------------------------------------------------
+// Wave K groups: 128x96, K-contiguous operands, four waves, one per SIMD.
+//
+// Every wave multiplies the whole tile over its own quarter of K (whole quads,
+// so every chunk stays whole) out of its own quarter of the LDS: what it reads
+// it has copied itself, so its K loop waits for its own copies only and has no
+// barrier.  The four sums are added in K order at the end, each wave a quarter
+// of the tile's rows.  A quad is walked as in the 256x256 kernel above: b's
+// fragments of 128 K in registers, a's a row of blocks ahead, four chunk MFMAs
+// and one sparse MFMA per block, the sums in accumulation registers.
+//
+// Against K groups that share a tile between four waves of 64x48 (pair form,
+// two waves per SIMD, a barrier per stage), each 64 K of a tile move 57 KiB
+// through the LDS (28 read, 28 written), not 86, which at 128 bytes a cycle
+// was more time than the stage's MFMAs.  Measured per call: Qwen2.5-1.5B down
+// 76.8 -> 67.2 us (840 TFLOP/s), q/o with a bias 20.4 -> 18.0.  On down the same
+// loop takes 48.6 us without its MFMAs (the copies: 224 KiB per quad and CU at
+// the address unit's 64 bytes a cycle are 3500 cycles) and 51.3 without its
+// copies (3840 cycles of MFMAs a quad), so neither bounds it alone; more bytes
+// in flight would need more LDS.
+//
+// LDS of a wave (40 KiB): b's quad (24 KiB) and a ring of four a row blocks
+// (4 KiB each).  Row i of a quad reads the fragments of row i + 1, copies row
+// i + 4 into its own slot (its fragments are in registers) and, in rows 1-4,
+// the next quad's b, whose fragments the last row reads as each column is done
+// with.  A copy has three rows (18 blocks, ~1500 cycles) to land.
+// ---------------------------------------------------------------------------
+template <int FM_, int FN_>
+struct WaveCfg {
+  static constexpr int FM = FM_, FN = FN_, BM = 16 * FM, BN = 16 * FN, KG = 4, T = 64 * KG;
+  static constexpr int QK = 4 * kChunk;                // K of a quad
+  static constexpr int SLOTS = 4, ROW = 16 * QK * 2;   // a's ring of row blocks, bytes each
+  static constexpr int B_AT = SLOTS * ROW, UBQ = 4 * FN;  // b's place in a ring; units a lane copies
+  static constexpr int RING = B_AT + BN * QK * 2, LDS = KG * RING;
+  static constexpr int PART = FM / KG * FN * 1024;     // a wave's FP32 sums of a quarter of the rows
+  static constexpr int FLAG_AT = (KG - 1) * PART;      // the tile flag, behind wave 0's inbox
+  static_assert(FM == 8 && FN % 2 == 0 && FN >= 6 && LDS <= 160 * 1024 && FLAG_AT + 4 <= RING, "schedule and LDS");
+  // store_any's view of it: wave w stores rows [32 w, 32 w + 32)
+  struct Store {
+    static constexpr int BM = 16 * FM_, BN = 16 * FN_, WAVES_M = KG, WAVES_N = 1, FM = FM_ / KG, FN = FN_;
+    static constexpr int WTM = 16 * FM, WTN = BN;
+  };
+  // copies a lane issues in row i: four of a, and FN of b in rows 1-4
+  static constexpr int copies(int i) { return 4 + (i >= 1 && i <= 4 ? FN : 0); }
+  // Copies issued after row i + 1's (issued in row i - 3) when row i, at its
+  // second block, reads its fragments; and after b's last (row 4) at row 7.
+  static constexpr int after_a(int i) {
+    return copies((i + FM - 2) % FM) + copies((i + FM - 1) % FM) + (i >= 1 && i <= 4 ? 1 : 0);
+  }
+  static constexpr int after_b() { return 1 + copies(5) + copies(6); }
+};
+
+// vmcnt(N), with no LDS read moved across: what the copies wrote is read next.
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Copies of a wave's quads, eight rows (a 64-K block, 128 bytes each) a unit,
+// in the layout of the 64-K stages: the swizzle differs between the first and
+// the second eight rows of a block of 16.  Rows past M (N) lie past the record
+// count (FastLoader's rule: the resource starts at the wave's first k, and rows
+// are at least K long), lanes past the wave's K range have the offset kOob.
+template <class C>
+struct WaveLoader {
+  i32x4 ra, rb;
+  int a_row, b_row;        // bytes per row
+  int k0[2];               // first k of the lane's unit, by parity of the unit's eight rows
+  int a_off[2], b_off[2];
+  int va[2][2], vb[2][2];  // lane offsets of the quad being copied: [64-K block][parity]
+
+  __device__ __forceinline__ void init(const Params& p, int64_t m0, int64_t n0, int64_t kbeg, int lane) {
+    ra = make_srd(p.a + (m0 * p.sam + kbeg));
+    rb = make_srd(p.b + (n0 * p.sbn + kbeg));
+    const int64_t ar = (p.M - m0) * p.sam * 2, br = (p.N - n0) * p.sbn * 2;
+    ra[2] = __builtin_amdgcn_readfirstlane((int)(ar < kOob ? ar : kOob));
+    rb[2] = __builtin_amdgcn_readfirstlane((int)(br < kOob ? br : kOob));
+    a_row = __builtin_amdgcn_readfirstlane((int)(p.sam * 2));
+    b_row = __builtin_amdgcn_readfirstlane((int)(p.sbn * 2));
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int row = 8 * h + (lane >> 3);
+      k0[h] = 8 * ((lane & 7) ^ kc_swz(row));
+      a_off[h] = row * a_row + 2 * k0[h];
+      b_off[h] = row * b_row + 2 * k0[h];
+    }
+  }
+  // Lane offsets of the quad at k = kq of the wave's kn.
+  __device__ __forceinline__ void at(int kq, int kn, const int (&off)[2], int (&v)[2][2]) const {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        v[s][h] = k0[h] + kStageK * s + kq < kn ? off[h] + 2 * (kStageK * s + kq) : kOob;
+  }
+  // Unit u (of 4) of a's row block i to its slot; unit u (of UBQ) of b.
+  __device__ __forceinline__ void a_unit(int i, int u, int lds) const {
+    lds_dma16_step(ra, lds + i % C::SLOTS * C::ROW + u * 1024, va[u / 2][u % 2], 16 * i * a_row);
+  }
+  __device__ __forceinline__ void b_unit(int u, int lds) const {
+    constexpr int PER = C::UBQ / 2;
+    lds_dma16_step(rb, lds + C::B_AT + u * 1024, vb[u / PER][u % 2], 16 * (u % PER / 2) * b_row);
+  }
+};
+
+// K loop of one wave over kn elements from kbeg (its ring at `ring`, LDS
+// address `lds`).
+template <class C, bool CHUNKED>
+__device__ __forceinline__ void k_loop_wave(const Params& p, int64_t m0, int64_t n0, int64_t kbeg, int kn,
+                                            const char LDS_AS* ring, int lds, int lane, f32x4 (&acc)[C::FM][C::FN]) {
+  if (kn <= 0) return;  // wave-uniform
+  constexpr int NB = C::FM * C::FN;
+  const char LDS_AS* bs = ring + C::B_AT;
+  const int r16 = lane & 15, g = lane >> 4;
+  auto frag_a = [&](int i, int c) __attribute__((always_inline)) {
+    return read_kc<C>(ring + i % C::SLOTS * C::ROW + (c >> 1) * (C::ROW / 2), r16, 4 * (c & 1) + g);
+  };
+  auto frag_b = [&](int j, int c) __attribute__((always_inline)) {
+    return read_kc<C>(bs + (c >> 1) * (C::BN * kStageK * 2), 16 * j + r16, 4 * (c & 1) + g);
+  };
+  WaveLoader<C> ld;
+  ld.init(p, m0, n0, kbeg, lane);
+  ld.at(0, kn, ld.a_off, ld.va);
+  ld.at(0, kn, ld.b_off, ld.vb);
+#pragma unroll
+  for (int u = 0; u < C::UBQ; ++u) ld.b_unit(u, lds);
+#pragma unroll
+  for (int i = 0; i < C::SLOTS; ++i)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) ld.a_unit(i, u, lds);
+  f16x8 bf[C::FN][4], af[2][4], sel;
+  f32x4 pr[4];   // as in k_loop_quad
+  f16x16 x[2];
+  int idx;
+  chunk_quad_selector(lane, sel, idx);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) pr[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  x[0] = x[1] = f16x16{};
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  wait_copies<(C::SLOTS - 1) * 4>();  // b, a's row 0
+#pragma unroll
+  for (int c = 0; c < 4; ++c) af[0][c] = frag_a(0, c);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) bf[j][c] = frag_b(j, c);
+  for (int kq = 0; kq < kn; kq += C::QK) {
+    // (past the wave's K every copy writes zeros, which no block multiplies)
+    ld.at(kq + C::QK, kn, ld.b_off, ld.vb);
+    static_for<NB>([&](auto block) __attribute__((always_inline)) {
+      constexpr int b = block, i = b / C::FN, j = b % C::FN;
+      if constexpr (i == C::FM - C::SLOTS && j == 0) ld.at(kq + C::QK, kn, ld.a_off, ld.va);
+      if constexpr (i == C::FM - 1 && j == 0) wait_copies<C::after_b()>();
+      if constexpr (j == 1) wait_copies<C::after_a(i)>();
+      if constexpr (j >= 1 && j <= 4) af[(i + 1) & 1][j - 1] = frag_a((i + 1) % C::FM, j - 1);
+      if constexpr (i >= 1 && i <= 4) ld.b_unit(C::FN * (i - 1) + j, lds);
+      if constexpr (j >= C::FN - 4) ld.a_unit((i + C::SLOTS) % C::FM, j - (C::FN - 4), lds);
+      if constexpr (CHUNKED) {
+        static_for<4>([&](auto chunk) __attribute__((always_inline)) {
+          constexpr int c = chunk, s = 4 * b + c;
+          __builtin_amdgcn_sched_barrier(0);
+          pr[s % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j][c], af[i & 1][c], zero, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          quad_round(pr[(s + 1) % 4], x[(c == 3 ? b : b + 1) & 1], (c + 1) % 4);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (c == 3) {
+            constexpr int sb = (b + NB - 1) % NB;
+            quad_sum(acc[sb / C::FN][sb % C::FN], sel, x[(b + 1) & 1], idx);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        });
+        if constexpr (i == C::FM - 1) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) bf[j][c] = frag_b(j, c);
+        }
+      } else {
+        static_for<4>([&](auto step) __attribute__((always_inline)) {
+          constexpr int c = 2 * (j & 1) + step / 2, col = (j & ~1) + step % 2;
+          __builtin_amdgcn_sched_barrier(0);
+          quad_mac(acc[i][col], bf[col][c], af[i & 1][c]);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (i == C::FM - 1) bf[col][c] = frag_b(col, c);
+        });
+      }
+    });
+  }
+  if constexpr (CHUNKED) {
+#pragma unroll
+    for (int c = 1; c < 4; ++c) quad_round(pr[c], x[1], c);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 7");  // conversions, then an MFMA the compiler does not see
+    __builtin_amdgcn_sched_barrier(0);
+    quad_sum(acc[C::FM - 1][C::FN - 1], sel, x[1], idx);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the sums' next readers
+  __builtin_amdgcn_sched_barrier(0);
+  wait_copies<0>();  // the copies past the K range
+}
+
+// The waves' sums of a tile, added in K order, ((S_0 + S_1) + S_2) + S_3: wave
+// w ends with rows [32 w, 32 w + 32).  Each wave leaves the other rows' sums in
+// their waves' inboxes (three parts in their rings, free after the first
+// barrier).  Clears the tile flag on the way.
+template <class C>
+__device__ __forceinline__ void wave_reduce(char LDS_AS* smem, int wave, int lane, const f32x4 (&acc)[C::FM][C::FN],
+                                            f32x4 (&sum)[C::FM / C::KG][C::FN]) {
+  constexpr int R = C::FM / C::KG;
+  __syncthreads();  // every wave is done with its ring
+  if (wave == 0 && lane == 0) *(int LDS_AS*)(smem + C::FLAG_AT) = 0;
+#pragma unroll
+  for (int w = 0; w < C::KG; ++w) {
+    if (w == wave) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < C::FN; ++j) sum[i][j] = quad_read(acc[R * w + i][j]);
+    } else {
+      char LDS_AS* to = smem + w * C::RING + (wave - (wave > w)) * C::PART + lane * 16;
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < C::FN; ++j) *(f32x4 LDS_AS*)(to + (i * C::FN + j) * 1024) = quad_read(acc[R * w + i][j]);
+    }
+  }
+  __syncthreads();
+  const char LDS_AS* in = smem + wave * C::RING + lane * 16;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) {
+      f32x4 v[C::KG - 1], own = sum[i][j];
+#pragma unroll
+      for (int h = 0; h < C::KG - 1; ++h) v[h] = *(const f32x4 LDS_AS*)(in + h * C::PART + (i * C::FN + j) * 1024);
+      f32x4 t = wave == 0 ? own : v[0];
+#pragma unroll
+      for (int h = 1; h < C::KG; ++h) t += h == wave ? own : h < wave ? v[h < C::KG - 1 ? h : 0] : v[h - 1];
+      sum[i][j] = t;
+    }
+}
+
+template <class C, bool CHUNKED, bool OUT32>
+__global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_wave(Params p) {
+  __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
+  char LDS_AS* smem = (char LDS_AS*)smem_raw;
+  typedef typename C::Store S;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char LDS_AS* ring = smem + wave * C::RING;
+  const int lds = __builtin_amdgcn_readfirstlane((int)(uint32_t)(size_t)ring);
+  const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n;
+  int64_t tm, tn;
+  group_m<uint32_t>(xcd_order<uint32_t>(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, &tm, &tn);
+  const int64_t m0 = tm * C::BM, n0 = tn * C::BN;
+  // this wave's quads: quads / 4, the first waves one more
+  const int quads = (int)((p.K + C::QK - 1) / C::QK), per = quads / C::KG, rem = quads % C::KG;
+  const int q0 = wave * per + (wave < rem ? wave : rem), nq = per + (wave < rem);
+  const int k0 = q0 * C::QK, kend = (q0 + nq) * C::QK;
+  const int kn = nq > 0 ? (kend < (int)p.K ? kend : (int)p.K) - k0 : 0;
+
+  f32x4 acc[C::FM][C::FN], sum[S::FM][S::FN];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  k_loop_wave<C, CHUNKED>(p, m0, n0, k0, kn, ring, lds, lane, acc);
+  const Bias<S> bias(p, n0, 0, lane);  // in flight under the reduction
+  wave_reduce<C>(smem, wave, lane, acc, sum);
+  store_any<S, OUT32, C::LDS>(p, ring, m0, n0, 0, wave, 0, lane, sum, bias);
+  if constexpr (CHUNKED && kRedo) {
+    bool bad = false;  // kernel.py:70-71
+#pragma unroll
+    for (int i = 0; i < S::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < S::FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bad |= !(__builtin_fabsf(sum[i][j][r]) < __builtin_inff());
+    int LDS_AS* word = (int LDS_AS*)(smem + C::FLAG_AT);
+    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *word = 1;
+    __syncthreads();
+    const int flag = *word;
+    if (p.flags && tid == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
+    if (__builtin_expect(flag, 0)) {
+      // redo the whole tile with FP32 accumulation (kernel.py:75-81), each
+      // wave over its own K range, then the same sums and stores
+      __syncthreads();  // every wave has read the flag, which wave 0's copies overwrite
+      clear();
+      k_loop_wave<C, false>(p, m0, n0, k0, kn, ring, lds, lane, acc);
+      wave_reduce<C>(smem, wave, lane, acc, sum);
+      store_any<S, OUT32, C::LDS>(p, ring, m0, n0, 0, wave, 0, lane, sum, bias);
+    }
+  }
+}
+
 // The redo launch of the deferred list (RedoList): the tiles a chunked
 // 256x256 launch flagged, each recomputed whole with FP32 accumulation
 // (kernel.py:75-81) as its four 128x128 quarters by four workgroups of C
@@ -2357,13 +2656,13 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 // ---------------------------------------------------------------------------
 // Tile configurations (ids are the F16ACC_TILE_* values of include/f16acc.h).
 //   id  tile     waves  wave tile  LDS ring      workgroups per CU (LDS)
-//   0   256x256  8      64x128     2 x 64 KiB    1
+//   0   256x256  4      128x128    160 KiB       1   (gemm_quad)
 //   1   256x128  8      64x64      3 x 48 KiB    1
 //   2   128x256  8      64x64      3 x 48 KiB    1
 //   3   128x128  4      64x64      2 x 32 KiB    2
 //   4   128x128  4      64x64      1 x 32 KiB    generic strided gather path
 //   5   64x64    4      32x32      2 x 16 KiB    4
-//   6   128x96   2 x 4  64x48      (2 + 3) x 28 KiB  1   (two K groups, split phases)
+//   6   128x96   4      128x96     4 x 40 KiB    1   (gemm_wave: each wave a quarter of K)
 //   7   64x32    4 x 2  32x32      2 x (2 + 3) x 12 KiB  1   (four K groups, split phases)
 //   8   256x288  8      64x144     2 x 68 KiB    1   (K-contiguous b)
 template <int BL> using Cfg1 = Cfg<256, 128, 4, 2, 3, BL>;
@@ -2371,14 +2670,11 @@ template <int BL> using Cfg2 = Cfg<128, 256, 2, 4, 3, BL>;
 template <int BL> using Cfg3 = Cfg<128, 128, 2, 2, 2, BL>;
 template <int BL> using Cfg5 = Cfg<64, 64, 2, 2, 2, BL, 4>;
 using CfgG = Cfg<128, 128, 2, 2, 2, kKC>;
-// K-group tiles, K-contiguous b only (a row-major b's k-rows of 12 or 4
-// units do not fit the transpose-read swizzle): 128x96 as two groups of 4
-// waves of 64x48, 64x32 as four groups of 2 waves of 32x32; split phases,
-// the early groups on two-stage rings, the late ones on three (140 KiB and
-// 120 KiB of LDS).  Measured against one phase (two-stage rings on 128x96,
-// three-stage on 64x32): Qwen2.5-1.5B q/o 18.46 -> 18.26 us, down 80.8 ->
-// 80.0, k/v 7.67 -> 7.35 (per call, same bits).
-using Cfg6 = Cfg<128, 96, 2, 2, 2, kKC, 2, 2, 3>;
+// 64x32 as four K groups of 2 waves of 32x32, K-contiguous b only (a row-major
+// b's k-rows of 4 units do not fit the transpose-read swizzle); split phases,
+// the early groups on two-stage rings, the late ones on three (120 KiB of LDS).
+// Measured against one phase (three-stage rings): Qwen2.5-1.5B k/v 7.67 -> 7.35
+// us (per call, same bits).
 using Cfg7 = Cfg<64, 32, 2, 1, 2, kKC, 2, 4, 3>;
 // 256x288: 256x256 widened by a ninth column block per wave (64x144), so
 // that 2048 x 8960 is one round of 256 tiles (8 x 32) instead of 280 256x256
@@ -2389,8 +2685,8 @@ struct TileInfo {
   int bm, bn, threads, per_cu;
 };
 constexpr TileInfo kTiles[F16ACC_NUM_TILES] = {
-    {256, 256, 512, 1}, {256, 128, 512, 1}, {128, 256, 512, 1}, {128, 128, 256, 2}, {128, 128, 256, 2},
-    {64, 64, 256, 4},   {128, 96, 512, 1},  {64, 32, 512, 1},   {256, 288, 512, 1}};
+    {256, 256, 256, 1}, {256, 128, 512, 1}, {128, 256, 512, 1}, {128, 128, 256, 2}, {128, 128, 256, 2},
+    {64, 64, 256, 4},   {128, 96, 256, 1},  {64, 32, 512, 1},   {256, 288, 512, 1}};
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -2590,7 +2886,7 @@ inline double rounds_288(int64_t n, int cus) {
 }
 
 // K-group tiles (kc: the operands allow them, a K-contiguous b on the fast
-// path), for small grids: 128x96 (two K groups) where its tiles fill more
+// path), for small grids: 128x96 where its tiles fill more
 // than half of the CUs in one round of one workgroup per CU, else 64x32 (four
 // K groups) where its tiles fit in one round at all.  Measured on MI355X:
 // Qwen2.5-1.5B k/v 2048x256x1536 7.96 us on 64x32 against 12.2 on 64x64
@@ -2857,6 +3153,23 @@ hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStre
   return hipGetLastError();
 }
 
+hipError_t launch_wave(const Params& p, int out32, int chunked, hipStream_t st) {
+  using C = WaveCfg<8, 6>;
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(C::T);
+  if (chunked) {
+    if (out32)
+      hipLaunchKernelGGL((gemm_wave<C, true, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_wave<C, true, false>), grid, block, 0, st, p);
+  } else {
+    if (out32)
+      hipLaunchKernelGGL((gemm_wave<C, false, true>), grid, block, 0, st, p);
+    else
+      hipLaunchKernelGGL((gemm_wave<C, false, false>), grid, block, 0, st, p);
+  }
+  return hipGetLastError();
+}
+
 template <class C>
 hipError_t launch_redo_list(const Params& p, int out32, int grid, hipStream_t st) {
   if (out32)
@@ -3085,7 +3398,7 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
       case 2: return (int)launch_fast<Cfg2>(q, ch.blayout, out32, chunked, st);
       case 3: return (int)launch_fast<Cfg3>(q, ch.blayout, out32, chunked, st);
       case 5: return (int)launch_fast<Cfg5>(q, ch.blayout, out32, chunked, st);
-      case 6: return (int)launch_cfg<Cfg6, kDma>(q, out32, chunked, st);
+      case 6: return (int)launch_wave(q, out32, chunked, st);
       case 7: return (int)launch_cfg<Cfg7, kDma>(q, out32, chunked, st);
       case 8: return (int)launch_cfg<Cfg8, kDma>(q, out32, chunked, st);
       default: return (int)launch_cfg<CfgG, kGather>(q, out32, chunked, st);

@@ -34,7 +34,7 @@ extern "C" {
 #define F16ACC_TILE_128x128 3
 #define F16ACC_TILE_GENERIC 4 /* 128x128, any strides, element gather */
 #define F16ACC_TILE_64x64 5   /* small grids: 4 waves of 32x32, 4 workgroups per CU */
-#define F16ACC_TILE_128x96_K2 6 /* two K groups of 4 waves of 64x48 splitting K inside the
+#define F16ACC_TILE_128x96_K2 6 /* K groups: four waves of 128x96, each a quarter of K inside the
                                    workgroup; K-contiguous b (else runs as 128x128) */
 #define F16ACC_TILE_64x32_K4 7  /* four K groups of 2 waves of 32x32 splitting K inside the
                                    workgroup; K-contiguous b (else runs as 64x64) */
