@@ -2128,7 +2128,8 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
 }
 
 // ---------------------------------------------------------------------------
-// Wave K groups: 128x96, K-contiguous operands, four waves, one per SIMD.
+// Wave K groups: 128x96 (K-contiguous operands) and 64x64 (either b; at most one
+// tile per CU, wave_64), four waves, one per SIMD.
 //
 // Every wave multiplies the whole tile over its own quarter of K (whole quads,
 // so every chunk stays whole) out of its own quarter of the LDS: what it reads
@@ -2148,35 +2149,50 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
 // copies (3840 cycles of MFMAs a quad), so neither bounds it alone; more bytes
 // in flight would need more LDS.
 //
-// LDS of a wave (40 KiB): b's quad (24 KiB) and a ring of four a row blocks
-// (4 KiB each).  Row i of a quad reads the fragments of row i + 1, copies row
-// i + 4 into its own slot (its fragments are in registers) and, in rows 1-4,
-// the next quad's b, whose fragments the last row reads as each column is done
-// with.  A copy has three rows (18 blocks, ~1500 cycles) to land.
+// LDS of a wave: b's quad (24 KiB on 128x96) and a ring of four a row blocks (4
+// KiB each).  Row i of a quad reads the fragments of row i + 1, copies row i + 4
+// into its own slot (its fragments are in registers) and, in the first half of
+// the rows but row 0, the next quad's b, whose fragments the last row reads as
+// each column is done with.  A copy of a has three rows (on 128x96 18 blocks,
+// ~1500 cycles) to land.
 // ---------------------------------------------------------------------------
-template <int FM_, int FN_>
+template <int FM_, int FN_, int BL_>
 struct WaveCfg {
-  static constexpr int FM = FM_, FN = FN_, BM = 16 * FM, BN = 16 * FN, KG = 4, T = 64 * KG;
+  static constexpr int FM = FM_, FN = FN_, BM = 16 * FM, BN = 16 * FN, KG = 4, T = 64 * KG, BL = BL_;
+  static constexpr int UB = BN / 8;                    // NC: units per k-row
   static constexpr int QK = 4 * kChunk;                // K of a quad
   static constexpr int SLOTS = 4, ROW = 16 * QK * 2;   // a's ring of row blocks, bytes each
   static constexpr int B_AT = SLOTS * ROW, UBQ = 4 * FN;  // b's place in a ring; units a lane copies
   static constexpr int RING = B_AT + BN * QK * 2, LDS = KG * RING;
   static constexpr int PART = FM / KG * FN * 1024;     // a wave's FP32 sums of a quarter of the rows
   static constexpr int FLAG_AT = (KG - 1) * PART;      // the tile flag, behind wave 0's inbox
-  static_assert(FM == 8 && FN % 2 == 0 && FN >= 6 && LDS <= 160 * 1024 && FLAG_AT + 4 <= RING, "schedule and LDS");
+  static_assert((FM == 8 || FM == SLOTS) && (FN == 4 || FN == 6), "the schedule's places");
+  static_assert(LDS <= 160 * 1024 && FLAG_AT + 4 <= RING, "LDS of a CU");
+  static_assert(BL == kKC || UB == 8, "an NC unit is eight k-rows, of one swizzle phase");
   // store_any's view of it: wave w stores rows [32 w, 32 w + 32)
   struct Store {
     static constexpr int BM = 16 * FM_, BN = 16 * FN_, WAVES_M = KG, WAVES_N = 1, FM = FM_ / KG, FN = FN_;
     static constexpr int WTM = 16 * FM, WTN = BN;
   };
-  // copies a lane issues in row i: four of a, and FN of b in rows 1-4
-  static constexpr int copies(int i) { return 4 + (i >= 1 && i <= 4 ? FN : 0); }
-  // Copies issued after row i + 1's (issued in row i - 3) when row i, at its
-  // second block, reads its fragments; and after b's last (row 4) at row 7.
+  // copies a lane issues in a block of row i: b's over rows 1 .. FM / 2, and a's
+  // four of a row from its third block on (by then the row's own fragments, whose
+  // slot they overwrite, have been multiplied)
+  static constexpr int B_ROWS = FM / 2;
+  static constexpr int b_copies(int i) { return i >= 1 && i <= B_ROWS ? 4 / B_ROWS : 0; }
+  static constexpr int A_COPIES = 4 / (FN - 2);
+  static constexpr int copies(int i) { return 4 + FN * b_copies(i); }
+  // Copies issued after row i + 1's (those in row i - 3) when row i, at its
+  // second block, reads its fragments (in the first quad's row 0: rows 2 and 3
+  // of the prologue); and after b's last when the last row reads b's.
   static constexpr int after_a(int i) {
-    return copies((i + FM - 2) % FM) + copies((i + FM - 1) % FM) + (i >= 1 && i <= 4 ? 1 : 0);
+    const int n = copies((i + FM - 2) % FM) + copies((i + FM - 1) % FM) + b_copies(i);
+    return i == 0 && n > 8 ? 8 : n;
   }
-  static constexpr int after_b() { return 1 + copies(5) + copies(6); }
+  static constexpr int after_b() {
+    int n = A_COPIES;
+    for (int i = B_ROWS + 1; i < FM - 1; ++i) n += copies(i);
+    return n;
+  }
 };
 
 // vmcnt(N), with no LDS read moved across: what the copies wrote is read next.
@@ -2207,13 +2223,28 @@ struct WaveLoader {
     ra[2] = __builtin_amdgcn_readfirstlane((int)(ar < kOob ? ar : kOob));
     rb[2] = __builtin_amdgcn_readfirstlane((int)(br < kOob ? br : kOob));
     a_row = __builtin_amdgcn_readfirstlane((int)(p.sam * 2));
-    b_row = __builtin_amdgcn_readfirstlane((int)(p.sbn * 2));
+    b_row = __builtin_amdgcn_readfirstlane((int)((C::BL == kKC ? p.sbn : p.sbk) * 2));
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int row = 8 * h + (lane >> 3);
       k0[h] = 8 * ((lane & 7) ^ kc_swz(row));
       a_off[h] = row * a_row + 2 * k0[h];
       b_off[h] = row * b_row + 2 * k0[h];
+    }
+    if (C::BL == kNC) {
+      const int krow = lane >> 3, ub = (lane & 7) ^ (nc_swz(krow) & (C::UB - 1));
+      b_off[0] = n0 + 8 * ub < p.N ? krow * b_row + ub * 16 : kOob;
+    }
+  }
+  // b's quad at k = kq of the wave's kn (an NC b's resource moves with it, its
+  // records the k-rows inside the range).
+  __device__ __forceinline__ void b_at(const Params& p, int64_t n0, int64_t kbeg, int kq, int kn) {
+    if (C::BL == kKC) {
+      at(kq, kn, b_off, vb);
+    } else {
+      const int krem = kn - kq < 0 ? 0 : kn - kq < C::QK ? kn - kq : C::QK;
+      rb = make_srd(p.b + ((kbeg + (krem > 0 ? kq : 0)) * p.sbk + n0));
+      rb[2] = __builtin_amdgcn_readfirstlane(krem * b_row);
     }
   }
   // Lane offsets of the quad at k = kq of the wave's kn.
@@ -2230,7 +2261,10 @@ struct WaveLoader {
   }
   __device__ __forceinline__ void b_unit(int u, int lds) const {
     constexpr int PER = C::UBQ / 2;
-    lds_dma16_step(rb, lds + C::B_AT + u * 1024, vb[u / PER][u % 2], 16 * (u % PER / 2) * b_row);
+    if (C::BL == kKC)
+      lds_dma16_step(rb, lds + C::B_AT + u * 1024, vb[u / PER][u % 2], 16 * (u % PER / 2) * b_row);
+    else
+      lds_dma16_step(rb, lds + C::B_AT + u * 1024, b_off[0], 8 * u * b_row);
   }
 };
 
@@ -2247,12 +2281,13 @@ __device__ __forceinline__ void k_loop_wave(const Params& p, int64_t m0, int64_t
     return read_kc<C>(ring + i % C::SLOTS * C::ROW + (c >> 1) * (C::ROW / 2), r16, 4 * (c & 1) + g);
   };
   auto frag_b = [&](int j, int c) __attribute__((always_inline)) {
+    if (C::BL == kNC) return read_nc<C>(bs, 16 * j, c, lane);
     return read_kc<C>(bs + (c >> 1) * (C::BN * kStageK * 2), 16 * j + r16, 4 * (c & 1) + g);
   };
   WaveLoader<C> ld;
   ld.init(p, m0, n0, kbeg, lane);
   ld.at(0, kn, ld.a_off, ld.va);
-  ld.at(0, kn, ld.b_off, ld.vb);
+  ld.b_at(p, n0, kbeg, 0, kn);
 #pragma unroll
   for (int u = 0; u < C::UBQ; ++u) ld.b_unit(u, lds);
 #pragma unroll
@@ -2277,15 +2312,21 @@ __device__ __forceinline__ void k_loop_wave(const Params& p, int64_t m0, int64_t
     for (int c = 0; c < 4; ++c) bf[j][c] = frag_b(j, c);
   for (int kq = 0; kq < kn; kq += C::QK) {
     // (past the wave's K every copy writes zeros, which no block multiplies)
-    ld.at(kq + C::QK, kn, ld.b_off, ld.vb);
+    ld.b_at(p, n0, kbeg, kq + C::QK, kn);
     static_for<NB>([&](auto block) __attribute__((always_inline)) {
       constexpr int b = block, i = b / C::FN, j = b % C::FN;
       if constexpr (i == C::FM - C::SLOTS && j == 0) ld.at(kq + C::QK, kn, ld.a_off, ld.va);
       if constexpr (i == C::FM - 1 && j == 0) wait_copies<C::after_b()>();
       if constexpr (j == 1) wait_copies<C::after_a(i)>();
-      if constexpr (j >= 1 && j <= 4) af[(i + 1) & 1][j - 1] = frag_a((i + 1) % C::FM, j - 1);
-      if constexpr (i >= 1 && i <= 4) ld.b_unit(C::FN * (i - 1) + j, lds);
-      if constexpr (j >= C::FN - 4) ld.a_unit((i + C::SLOTS) % C::FM, j - (C::FN - 4), lds);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)  // the next row's fragments
+        if (j == (C::FN == 4 && c > 0 ? c : c + 1)) af[(i + 1) & 1][c] = frag_a((i + 1) % C::FM, c);
+#pragma unroll
+      for (int e = 0; e < C::b_copies(i); ++e) ld.b_unit(C::b_copies(i) * (C::FN * (i - 1) + j) + e, lds);
+      if constexpr (j >= 2) {
+#pragma unroll
+        for (int e = 0; e < C::A_COPIES; ++e) ld.a_unit((i + C::SLOTS) % C::FM, C::A_COPIES * (j - 2) + e, lds);
+      }
       if constexpr (CHUNKED) {
         static_for<4>([&](auto chunk) __attribute__((always_inline)) {
           constexpr int c = chunk, s = 4 * b + c;
@@ -2370,7 +2411,9 @@ __device__ __forceinline__ void wave_reduce(char LDS_AS* smem, int wave, int lan
     }
 }
 
-template <class C, bool CHUNKED, bool OUT32>
+// R: the tile's configuration whose K loop redoes an overflowing tile, so that
+// it equals the FP32 mode of that tile (WaveCfg itself where that runs here).
+template <class C, class R, bool CHUNKED, bool OUT32>
 __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_wave(Params p) {
   __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
   char LDS_AS* smem = (char LDS_AS*)smem_raw;
@@ -2415,13 +2458,27 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
     const int flag = *word;
     if (p.flags && tid == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
     if (__builtin_expect(flag, 0)) {
-      // redo the whole tile with FP32 accumulation (kernel.py:75-81), each
-      // wave over its own K range, then the same sums and stores
+      // redo the whole tile with FP32 accumulation (kernel.py:75-81)
+      wait_vm0();       // the first store is done: other threads may store over it
       __syncthreads();  // every wave has read the flag, which wave 0's copies overwrite
-      clear();
-      k_loop_wave<C, false>(p, m0, n0, k0, kn, ring, lds, lane, acc);
-      wave_reduce<C>(smem, wave, lane, acc, sum);
-      store_any<S, OUT32, C::LDS>(p, ring, m0, n0, 0, wave, 0, lane, sum, bias);
+      if constexpr (std::is_same<C, R>::value) {
+        clear();
+        k_loop_wave<C, false>(p, m0, n0, k0, kn, ring, lds, lane, acc);
+        wave_reduce<C>(smem, wave, lane, acc, sum);
+        store_any<S, OUT32, C::LDS>(p, ring, m0, n0, 0, wave, 0, lane, sum, bias);
+      } else {
+        static_assert(R::T == C::T && R::BM == C::BM && R::BN == C::BN && R::RINGS <= C::LDS, "the same tile");
+        const int wm = wave / R::WAVES_N, wn = wave % R::WAVES_N;
+        f32x4 all[R::FM][R::FN];
+#pragma unroll
+        for (int i = 0; i < R::FM; ++i)
+#pragma unroll
+          for (int j = 0; j < R::FN; ++j) all[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        FastLoader<R> fl;
+        fl.init(p, m0, n0, tid);
+        k_loop_fast<R, false>(p, m0, n0, 0, p.K, smem, fl, wave, wm, wn, lane, all);
+        store_any<R, OUT32, C::LDS>(p, smem, m0, n0, wave, wm, wn, lane, all, Bias<R>(p, n0, wn, lane));
+      }
     }
   }
 }
@@ -3153,19 +3210,19 @@ hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStre
   return hipGetLastError();
 }
 
+template <class C, class R>
 hipError_t launch_wave(const Params& p, int out32, int chunked, hipStream_t st) {
-  using C = WaveCfg<8, 6>;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(C::T);
   if (chunked) {
     if (out32)
-      hipLaunchKernelGGL((gemm_wave<C, true, true>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_wave<C, R, true, true>), grid, block, 0, st, p);
     else
-      hipLaunchKernelGGL((gemm_wave<C, true, false>), grid, block, 0, st, p);
-  } else {
+      hipLaunchKernelGGL((gemm_wave<C, R, true, false>), grid, block, 0, st, p);
+  } else if constexpr (std::is_same<C, R>::value) {
     if (out32)
-      hipLaunchKernelGGL((gemm_wave<C, false, true>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_wave<C, R, false, true>), grid, block, 0, st, p);
     else
-      hipLaunchKernelGGL((gemm_wave<C, false, false>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_wave<C, R, false, false>), grid, block, 0, st, p);
   }
   return hipGetLastError();
 }
@@ -3252,6 +3309,20 @@ inline bool deferred_redo(const Choice& ch, int64_t M, int64_t N, int64_t K, int
     return false;
   const int64_t tiles = cdiv(M, 256) * cdiv(N, 256);
   return tiles <= cus && tiles <= kRedoMax;
+}
+
+// 64x64 tiles of at most one per CU, chunked: four waves, each a quarter of K
+// (gemm_wave), from a quad a wave on.  One workgroup of the ordinary kernel
+// alone on its CU waits out a copy's latency every 64 K: 1024 x 1024 x 1024 fp32
+// out 10.9 -> 8.75 us a call.  Two or more workgroups on a CU hide each other's
+// waits and keep the ordinary kernel (2048 x 1024 x 1024: 10.3 us against 13.3
+// in K groups; 1536 x 1024 x 2048: 17.4 against 19.7), as do the second launch
+// of a cut (one grid's summation order) and a row-major b whose 128 k-rows pass
+// 32-bit offsets.
+inline bool wave_64(const Choice& ch, const Params& p, int cus) {
+  return ch.tile == F16ACC_TILE_64x64 && ch.family == F16ACC_FAMILY_FAST && p.tiles_m * p.tiles_n <= cus &&
+         p.K >= 4 * 4 * kChunk &&
+         (ch.blayout == kKC || (int64_t)4 * kChunk * p.sbk * 2 + 2 * 64 < kOob);
 }
 
 // Split redo (F16ACC_SPLIT_REDO builds only, for the benchmark): the
@@ -3386,6 +3457,9 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
   if (p.tiles_m * p.tiles_n * p.splits > 0x7fffffff) return F16ACC_E_UNSUPPORTED;
   const int out32 = out_dtype == F16ACC_OUT_F32;
   hipStream_t st = (hipStream_t)stream;
+  // (a forced 64x64 runs as the table's pick does, where the table picks it)
+  const bool wave64 = chunked && kgroups && wave_64(ch, p, cu_count()) &&
+                      (forced_tile < 0 || choose(M, N, K, sam, sak, sbk, sbn, a, b, -1).tile == F16ACC_TILE_64x64);
   auto launch = [&](const Params& q) -> int {
     if (ch.family == F16ACC_FAMILY_REG)  // 64x64 only with a K-contiguous b (choose)
       return ch.tile == F16ACC_TILE_64x64 ? (int)launch_cfg<Cfg5<kKC>, kReg>(q, out32, chunked, st)
@@ -3397,8 +3471,12 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
       case 1: return (int)launch_fast<Cfg1>(q, ch.blayout, out32, chunked, st);
       case 2: return (int)launch_fast<Cfg2>(q, ch.blayout, out32, chunked, st);
       case 3: return (int)launch_fast<Cfg3>(q, ch.blayout, out32, chunked, st);
-      case 5: return (int)launch_fast<Cfg5>(q, ch.blayout, out32, chunked, st);
-      case 6: return (int)launch_wave(q, out32, chunked, st);
+      case 5:
+        if (wave64)
+          return ch.blayout == kKC ? (int)launch_wave<WaveCfg<4, 4, kKC>, Cfg5<kKC>>(q, out32, chunked, st)
+                                   : (int)launch_wave<WaveCfg<4, 4, kNC>, Cfg5<kNC>>(q, out32, chunked, st);
+        return (int)launch_fast<Cfg5>(q, ch.blayout, out32, chunked, st);
+      case 6: return (int)launch_wave<WaveCfg<8, 6, kKC>, WaveCfg<8, 6, kKC>>(q, out32, chunked, st);
       case 7: return (int)launch_cfg<Cfg7, kDma>(q, out32, chunked, st);
       case 8: return (int)launch_cfg<Cfg8, kDma>(q, out32, chunked, st);
       default: return (int)launch_cfg<CfgG, kGather>(q, out32, chunked, st);

@@ -1,10 +1,12 @@
-"""The 128x96 K-group kernel (each wave a quarter of K) where its schedule can
-go wrong: K around whole quads and around one quad per wave, ragged tiles,
-both output types and modes."""
+"""The K-quarter kernel (each wave a quarter of K: 128x96 from K = 1536, 64x64
+with at most one tile per CU) where its schedule can go wrong: K around whole
+quads and around the rules' lines, ragged tiles, both output types, an overflow
+in any quarter."""
 
 import pytest
 import torch
 
+import f16acc_amd as f16acc
 from f16acc_amd.kernel import mm_flags, mm_tile, tile_config
 from oracle import chunk32
 
@@ -17,7 +19,7 @@ def rnd(shape, seed):
 
 
 @pytest.mark.parametrize("M, N", [(128, 96), (129, 97), (120, 200)])
-@pytest.mark.parametrize("K", [8, 120, 128, 136, 384, 504, 512, 520, 640, 1032, 1160, 2568])
+@pytest.mark.parametrize("K", [8, 136, 1160, 1528, 1536, 1544, 1640, 1664, 1928, 2040, 2048, 2056, 2568])
 def test_quads_per_wave_against_the_oracle(M, N, K):
     a, w = rnd((M, K), 7 + K), rnd((N, K), 8 + K)
     ga, gb = a.cuda(), w.cuda().t()
@@ -31,3 +33,69 @@ def test_quads_per_wave_against_the_oracle(M, N, K):
     assert torch.equal(mm_tile(ga, gb, TILE), c32.half())
     full = mm_tile(ga, gb, TILE, torch.float32, chunked=False)
     assert chunk32.rel(full.cpu(), (a.float() @ w.t().float()).double()) < 1e-5
+
+
+def picks_64(a, b):
+    cfg = tile_config(a, b)
+    assert cfg["tile"] == "64x64" and cfg["tiles_m"] * cfg["tiles_n"] <= 256
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M, N, K", [(1024, 1024, 512), (1024, 1024, 1024), (1000, 1016, 520), (961, 1024, 648),
+                                     (1024, 968, 1160), (1023, 1000, 1544)])
+def test_64x64_in_k_quarters_against_one_wave_group(M, N, K, b_t):
+    """At most one 64x64 tile per CU runs in wave K groups; 128x128 sums K in
+    order.  The same rounded chunks in another FP32 order (sums
+    below 2^8 of values of at most 11 bits: at most a few ulps of FP32 apart)."""
+    a, w = rnd((M, K), 31).cuda(), rnd((N, K), 32).cuda()
+    b = w.t() if b_t else w.t().contiguous()
+    picks_64(a, b)
+    c, flags = mm_flags(a, b, torch.float32)
+    one = mm_tile(a, b, "128x128", torch.float32)
+    off = (c - one).abs()
+    # an element may also hold a partial that summed to the other side of a tie
+    assert int(flags.sum()) == 0 and float((off > 1e-4).float().mean()) < 1e-3 * K / 32 and float(off.max()) < 2 ** -4
+    assert torch.equal(f16acc.mm(a, b), c.half()) and torch.equal(mm_tile(a, b, "64x64", torch.float32), c)
+
+
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("quarter", range(4))
+def test_64x64_redoes_an_overflow_in_any_quarter(quarter, b_t):
+    """The overflow closed form (chunk sums past 65504 that cancel: exactly 100
+    in FP32) in one wave's K range, the other ranges zero there."""
+    M = N = 1024
+    K = 512
+    a, b = rnd((M, K), 33), rnd((K, N), 34)
+    r0, c0, k0 = 64 * 5 + 20, 64 * 11 + 40, 128 * quarter
+    a[r0:r0 + 10, :] = 100.0
+    b[:, c0:c0 + 10] = 0.0
+    for q, v in enumerate((30.0, -30.0, 30.0, -30.0)):
+        b[k0 + 32 * q:k0 + 32 * q + 32, c0:c0 + 10] = v
+    b[k0 + 127, c0:c0 + 10] = -29.0
+    ga, gb = a.cuda(), b.t().contiguous().cuda().t() if b_t else b.cuda()
+    picks_64(ga, gb)
+    c, flags = mm_flags(ga, gb, torch.float32)
+    assert int(flags.sum()) == 1 and flags[5, 11] == 1
+    assert bool((c[r0:r0 + 10, c0:c0 + 10] == 100.0).all())
+    # redone whole in FP32: the bits of that mode
+    full = mm_tile(ga, gb, "64x64", torch.float32, chunked=False)
+    assert torch.equal(c[320:384, 704:768], full[320:384, 704:768])
+
+
+@pytest.mark.parametrize("quarter", range(4))
+def test_128x96_redoes_an_overflow_in_any_quarter(quarter):
+    """The same closed form on tile (1, 1) of 128x96 at K = 1536."""
+    M, N, K = 300, 250, 1536
+    a, w = rnd((M, K), 35), rnd((N, K), 36)
+    r0, c0, k0 = 128 + 70, 96 + 60, 384 * quarter + 128
+    a[r0:r0 + 10, :] = 100.0
+    w[c0:c0 + 10, :] = 0.0
+    for q, v in enumerate((30.0, -30.0, 30.0, -30.0)):
+        w[c0:c0 + 10, k0 + 32 * q:k0 + 32 * q + 32] = v
+    w[c0:c0 + 10, k0 + 127] = -29.0
+    ga, gb = a.cuda(), w.cuda().t()
+    c, flags = mm_flags(ga, gb, torch.float32, tile=TILE)
+    assert int(flags.sum()) == 1 and flags[1, 1] == 1
+    assert bool((c[r0:r0 + 10, c0:c0 + 10] == 100.0).all())
+    full = mm_tile(ga, gb, TILE, torch.float32, chunked=False)
+    assert torch.equal(c[128:256, 96:192], full[128:256, 96:192])
