@@ -2719,7 +2719,8 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 //   3   128x128  4      64x64      2 x 32 KiB    2
 //   4   128x128  4      64x64      1 x 32 KiB    generic strided gather path
 //   5   64x64    4      32x32      2 x 16 KiB    4
-//   6   128x96   4      128x96     4 x 40 KiB    1   (gemm_wave: each wave a quarter of K)
+//   6   128x96   4      128x96     4 x 40 KiB    1   (gemm_wave: each wave a quarter of K; short K: two K
+//                                                    groups of 2 x 2 waves of 64x48)
 //   7   64x32    4 x 2  32x32      2 x (2 + 3) x 12 KiB  1   (four K groups, split phases)
 //   8   256x288  8      64x144     2 x 68 KiB    1   (K-contiguous b)
 template <int BL> using Cfg1 = Cfg<256, 128, 4, 2, 3, BL>;
@@ -2727,11 +2728,13 @@ template <int BL> using Cfg2 = Cfg<128, 256, 2, 4, 3, BL>;
 template <int BL> using Cfg3 = Cfg<128, 128, 2, 2, 2, BL>;
 template <int BL> using Cfg5 = Cfg<64, 64, 2, 2, 2, BL, 4>;
 using CfgG = Cfg<128, 128, 2, 2, 2, kKC>;
-// 64x32 as four K groups of 2 waves of 32x32, K-contiguous b only (a row-major
-// b's k-rows of 4 units do not fit the transpose-read swizzle); split phases,
-// the early groups on two-stage rings, the late ones on three (120 KiB of LDS).
-// Measured against one phase (three-stage rings): Qwen2.5-1.5B k/v 7.67 -> 7.35
-// us (per call, same bits).
+// K-group tiles of several waves a group, K-contiguous b only (a row-major b's
+// k-rows of 12 or 4 units do not fit the transpose-read swizzle): 128x96 at a
+// short K (wave_128x96) as two groups of 4 waves of 64x48, 64x32 as four groups of
+// 2 waves of 32x32; split phases, the early groups on two-stage rings, the late
+// ones on three (140 KiB and 120 KiB of LDS).  Measured against one phase:
+// Qwen2.5-1.5B k/v 7.67 -> 7.35 us (per call, same bits).
+using Cfg6 = Cfg<128, 96, 2, 2, 2, kKC, 2, 2, 3>;
 using Cfg7 = Cfg<64, 32, 2, 1, 2, kKC, 2, 4, 3>;
 // 256x288: 256x256 widened by a ninth column block per wave (64x144), so
 // that 2048 x 8960 is one round of 256 tiles (8 x 32) instead of 280 256x256
@@ -3311,6 +3314,13 @@ inline bool deferred_redo(const Choice& ch, int64_t M, int64_t N, int64_t K, int
   return tiles <= cus && tiles <= kRedoMax;
 }
 
+// 128x96 in wave K groups (gemm_wave) from three quads a wave on: below, filling
+// four rings and adding four sums cost more than the loop saves.
+// Per call against two K groups, 2048 x 1536: K = 512 10.5 us against 9.6, 768
+// 12.7 against 11.4, 1280 15.9 against 15.2, 1536 17.5 against 17.7, 2048 20.7
+// against 22.1 (1536 x 1536 and 1407 x 2005 cross at the same K).
+inline bool wave_128x96(const Params& p) { return p.K >= 3 * 4 * 4 * kChunk; }
+
 // 64x64 tiles of at most one per CU, chunked: four waves, each a quarter of K
 // (gemm_wave), from a quad a wave on.  One workgroup of the ordinary kernel
 // alone on its CU waits out a copy's latency every 64 K: 1024 x 1024 x 1024 fp32
@@ -3476,7 +3486,9 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
           return ch.blayout == kKC ? (int)launch_wave<WaveCfg<4, 4, kKC>, Cfg5<kKC>>(q, out32, chunked, st)
                                    : (int)launch_wave<WaveCfg<4, 4, kNC>, Cfg5<kNC>>(q, out32, chunked, st);
         return (int)launch_fast<Cfg5>(q, ch.blayout, out32, chunked, st);
-      case 6: return (int)launch_wave<WaveCfg<8, 6, kKC>, WaveCfg<8, 6, kKC>>(q, out32, chunked, st);
+      case 6:
+        return wave_128x96(q) ? (int)launch_wave<WaveCfg<8, 6, kKC>, WaveCfg<8, 6, kKC>>(q, out32, chunked, st)
+                              : (int)launch_cfg<Cfg6, kDma>(q, out32, chunked, st);
       case 7: return (int)launch_cfg<Cfg7, kDma>(q, out32, chunked, st);
       case 8: return (int)launch_cfg<Cfg8, kDma>(q, out32, chunked, st);
       default: return (int)launch_cfg<CfgG, kGather>(q, out32, chunked, st);
