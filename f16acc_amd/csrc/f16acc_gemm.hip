@@ -94,7 +94,7 @@ constexpr bool kRedo = !F16ACC_NO_REDO;
 constexpr bool kSplitRedo = F16ACC_SPLIT_REDO && kRedo;
 
 // F16ACC_NO_PERSISTENT=1 runs multi-round shapes on the one-tile-per-
-// workgroup grid instead of the persistent kernel (gemm_persistent); only
+// workgroup grid instead of gemm_quad's walk over them; only
 // the benchmark's A/B of the two builds loads it (same bits either way).
 #ifndef F16ACC_NO_PERSISTENT
 #define F16ACC_NO_PERSISTENT 0
@@ -285,7 +285,7 @@ struct Cfg {
   // the group reduction parks groups 1..KG-1's sums in the (free) rings
   static_assert((KG - 1) * BM * BN * 4 <= RINGS, "group sums must fit the LDS rings");
   // Split-K partial stores are compiled only into tiles of 64x64 per wave:
-  // at 64x128 per wave the chunked kernel already uses ~240 of its 256
+  // at 64x144 per wave the chunked kernel already uses all of its 256
   // registers, and the extra path would make it spill.  K-group tiles split
   // inside the workgroup instead.
   static constexpr bool SPLITTABLE = FM * FN <= 16 && KG == 1;
@@ -837,7 +837,7 @@ __device__ __forceinline__ void group_reduce(char LDS_AS* smem, int g, int ltid,
 // The fast path's K loop over [kbeg, kend) for this thread's K group, then
 // the group reduction: group 0 ends with the tile's sum.
 
-// Chunked K loop of the 64x128-per-wave tiles (256x256, 256x288), with the
+// Chunked K loop of the 64x144-per-wave tile (256x288), with the
 // stage barrier moved from a stage's start to before its last column: a
 // two-stage ring, where a wave that reaches the barrier has read every
 // fragment of stage s (its last b column is in registers) and has its own
@@ -851,8 +851,7 @@ __device__ __forceinline__ void group_reduce(char LDS_AS* smem, int g, int ltid,
 // (spread over its first half, as k_loop_fast does, they left too little
 // time where the operands come from HBM: the lm_head shape ran 3 % slower).
 // Same operations in the same order as k_loop_fast (same bits); measured
-// 0.9-1.4 % faster on 4096^3, 8192^3 and Qwen gate/up, level on the lm_head
-// shape.  (FP32 accumulation keeps k_loop_fast: there this form ran 2-6 %
+// 0.9-1.4 % faster on Qwen2.5-1.5B gate/up.  (FP32 accumulation keeps k_loop_fast: there this form ran 2-6 %
 // slower.)
 template <class C>
 __device__ __forceinline__ void k_loop_cross(const Params& p, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
