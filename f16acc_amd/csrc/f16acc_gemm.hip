@@ -1866,10 +1866,11 @@ __device__ __forceinline__ void k_loop_quad(const Params& p, int64_t m0, int64_t
 }
 
 // Whether a wave's sub-tile is stored whole: inside c, rows contiguous and 16-
-// byte aligned, offsets in 32 bits (C::stores() buffer stores).
+// byte aligned, offsets in 32 bits (C::stores() buffer stores).  Those offsets
+// are unsigned: rows that go backwards (scm < 0) are stored through pointers.
 template <class C, bool OUT32>
 __device__ __forceinline__ bool quad_whole(const Params& p, int64_t m0, int64_t n0, int wm, int wn) {
-  return p.vec_store && p.M - m0 >= (wm + 1) * C::WTM && p.N - n0 >= (wn + 1) * C::WTN &&
+  return p.vec_store && p.M - m0 >= (wm + 1) * C::WTM && p.N - n0 >= (wn + 1) * C::WTN && p.scm >= 0 &&
          C::WTM * p.scm * (OUT32 ? 4 : 2) < kOob;
 }
 

@@ -17,7 +17,7 @@ import torch
 
 import f16acc_amd as f16acc
 from f16acc_amd import _lib
-from f16acc_amd.kernel import mm_flags, tile_config
+from f16acc_amd.kernel import mm_flags, mm_tile, tile_config
 from oracle import chunk32
 
 pytestmark = pytest.mark.gpu
@@ -943,6 +943,31 @@ def test_c_abi_writes_any_output_strides(shape, out_dtype):
         view(written.view(-1)).fill_(True)
         untouched = torch.cat([buf[:32], body[~written], buf[32 + numel:]])
         assert bool((untouched == sentinel).all()), (name, shape, out_dtype)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("tile", ALL_TILES)
+def test_c_abi_writes_reversed_rows_and_columns(tile, out_dtype):
+    """Negative c strides (c a flipped view, its pointer at the last row or
+    column): 300 x 520 holds whole and partial wave sub-tiles of every tile, rows
+    16-byte aligned.  The bits of the contiguous result, nothing else
+    written."""
+    from f16acc_amd import _lib
+
+    M, N, K = 300, 520, 160
+    a, b = rnd((M, K), 72).cuda(), rnd((N, K), 73).cuda().t()
+    want = mm_tile(a, b, tile, out_dtype)
+    out = _lib.OUT_F32 if out_dtype == torch.float32 else _lib.OUT_F16
+    for rows, cols in ((True, False), (False, True), (True, True)):
+        buf = torch.full((M * N + 64,), -7.0, device="cuda", dtype=out_dtype)
+        body = buf[32:32 + M * N]
+        first = (M - 1) * N * rows + (N - 1) * cols
+        _lib.check(_lib.gemm_tile(a.data_ptr(), b.data_ptr(), body[first:].data_ptr(), None, M, N, K, K, 1, 1, K,
+                                  -N if rows else N, -1 if cols else 1, out, 1,
+                                  torch.cuda.current_stream().cuda_stream, _lib.TILES.index(tile)))
+        c = body.view(M, N).flip([d for d, on in ((0, rows), (1, cols)) if on])
+        assert torch.equal(c, want), (tile, rows, cols)
+        assert bool((buf[:32] == -7.0).all()) and bool((buf[32 + M * N:] == -7.0).all())
 
 
 def test_launch_stream_is_the_current_torch_stream():
