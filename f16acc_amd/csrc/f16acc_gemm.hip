@@ -2010,11 +2010,10 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
 // tile order of a whole grid.  The next tile's first quad is copied before
 // this tile is stored, and the stores drain under its K loop.  An overflowing
 // tile (kernel.py:70-81) is listed for the redo launch (p.list) or redone
-// here, whole, with FP32 accumulation, as its four 128x128 quarters (C3): every
-// element sums the same products in the same order as the FP32 mode.
-template <class C, class C3, bool CHUNKED, bool OUT32>
+// here: the same tile once more, over all of K, with the FP32 mode's own loop
+// (so with its bits).
+template <class C, bool CHUNKED, bool OUT32>
 __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_quad(Params p) {
-  static_assert(C3::T == C::T && C3::BM * 2 == C::BM && C3::BN * 2 == C::BN && C3::RINGS <= C::LDS, "quarters");
   __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
   char LDS_AS* smem = (char LDS_AS*)smem_raw;
   const int tid = threadIdx.x;
@@ -2027,6 +2026,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
   int64_t tm, tn;
   group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &tm, &tn);
   bool issued = false;
+  [[maybe_unused]] bool redo = false;  // this pass redoes the tile of the last one
   int since = kNothing;
   for (;;) {
     const int64_t m0 = tm * C::BM, n0 = tn * C::BN;
@@ -2045,7 +2045,10 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
       ld.init(p, m0, n0, tid_t);
       if (!issued) ld.first(p, m0, n0, lds);
       constexpr int kStores = C::stores(OUT32) < 63 ? C::stores(OUT32) : 63;
-      k_loop_quad<C, CHUNKED, kStores>(p, m0, n0, smem, ld, lds, wm, wn, lane, since, acc);
+      if (CHUNKED && kRedo && redo)
+        k_loop_quad<C, false, kStores>(p, m0, n0, smem, ld, lds, wm, wn, lane, since, acc);
+      else
+        k_loop_quad<C, CHUNKED, kStores>(p, m0, n0, smem, ld, lds, wm, wn, lane, since, acc);
     }
     f16x8 bias[4] = {};  // this lane's columns: 16 j + 4 (lane / 16) + r
     if (p.bias) {
@@ -2058,7 +2061,7 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
       // waited for here: behind the next tile's copies a wait would include them
       asm volatile("" : "+v"(bias[0]), "+v"(bias[1]), "+v"(bias[2]), "+v"(bias[3]));
     }
-    t += gridDim.x;  // (no wrap: both are below 2^31)
+    if (!redo) t += gridDim.x;  // (no wrap: both are below 2^31)
     const bool next = t < tiles && p.K > 0;
     int64_t ntm = 0, ntn = 0;
     if (t < tiles) group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &ntm, &ntn);
@@ -2073,51 +2076,44 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
     [[maybe_unused]] const bool bad = p.bias ? quad_store<C, OUT32, true>(p, slice, m0, n0, wm, wn, lane, acc, bias)
                             : quad_store<C, OUT32, false>(p, slice, m0, n0, wm, wn, lane, acc, bias);
     if constexpr (CHUNKED && kRedo) {
-      // tile flag: one word at the start of the staging area
-      int LDS_AS* word = (int LDS_AS*)(smem + C::STAGE_AT);
-      if (tid_t == 0) *word = 0;  // wave 0's staging is done with it
-      __syncthreads();
-      if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *word = 1;
-      __syncthreads();
-      const int flag = *word;
-      if (p.flags && tid_t == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
-      if (__builtin_expect(flag, 0) && !(kSplitRedo && p.defer_redo)) {
-        bool here = true;
+      if (redo) {
+        redo = false;  // stored; the flag stays as it was
+      } else {
+        // tile flag: one word at the start of the staging area
+        int LDS_AS* word = (int LDS_AS*)(smem + C::STAGE_AT);
+        if (tid_t == 0) *word = 0;  // wave 0's staging is done with it
         __syncthreads();
-        if (p.list) {
-          // deferred: a list that is full (or not zeroed) leaves the redo here
-          if (tid_t == 0) {
-            const int at = atomicAdd(&p.list->alloc, 1);
-            const bool listed = at >= 0 && at < kRedoMax;
-            if (listed) {
-              store_agent(&p.list->items[at], (int)(tm * p.tiles_n + tn));
+        if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) *word = 1;
+        __syncthreads();
+        const int flag = __builtin_amdgcn_readfirstlane(*word);
+        if (p.flags && tid_t == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
+        if (__builtin_expect(flag, 0) && !(kSplitRedo && p.defer_redo)) {
+          redo = true;
+          __syncthreads();
+          if (p.list) {
+            // deferred: a list that is full (or not zeroed) leaves the redo here
+            if (tid_t == 0) {
+              const int at = atomicAdd(&p.list->alloc, 1);
+              const bool listed = at >= 0 && at < kRedoMax;
+              if (listed) {
+                store_agent(&p.list->items[at], (int)(tm * p.tiles_n + tn));
 #pragma unroll
-              for (int j = 0; j < kLines; ++j) atomicAdd(&p.list->line[j].word, 1ull);
+                for (int j = 0; j < kLines; ++j) atomicAdd(&p.list->line[j].word, 1ull);
+              }
+              *word = listed ? 2 : 1;
             }
-            *word = listed ? 2 : 1;
+            __syncthreads();
+            redo = __builtin_amdgcn_readfirstlane(*word) != 2;
           }
-          __syncthreads();
-          here = *word != 2;
-        }
-        if (here) {
-          wait_vm0();  // the next tile's copies have landed: the redo takes their place
-          __syncthreads();
-          for (int quarter = 0; quarter < 4; ++quarter) {
-            const int64_t qm = m0 + quarter / 2 * C3::BM, qn = n0 + quarter % 2 * C3::BN;
-            if (qm >= p.M || qn >= p.N) continue;
-            f32x4 sum[C3::FM][C3::FN];
-#pragma unroll
-            for (int i = 0; i < C3::FM; ++i)
-#pragma unroll
-              for (int j = 0; j < C3::FN; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            FastLoader<C3> fl;
-            fl.init(p, qm, qn, tid_t);
-            k_loop_fast<C3, false>(p, qm, qn, 0, p.K, smem, fl, wave, wm, wn, lane, sum);
-            store_any<C3, OUT32, C::LDS>(p, smem, qm, qn, wave, wm, wn, lane, sum, Bias<C3>(p, qn, wn, lane));
-            __syncthreads();  // staging reads done before the next quarter's copies
+          if (redo) {
+            // the next tile's copies, landed by now, give way to this tile's
+            // and are made again behind its loop; its stores follow these
+            wait_vm0();
+            __syncthreads();
+            issued = false;
+            since = kNothing;
+            continue;
           }
-          issued = false;
-          since = kNothing;
         }
       }
     }
@@ -3201,14 +3197,14 @@ hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStre
   const dim3 grid((unsigned)(persistent ? cus : tiles)), block(C::T);
   if (chunked) {
     if (out32)
-      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true, true>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_quad<C, true, true>), grid, block, 0, st, p);
     else
-      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, true, false>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_quad<C, true, false>), grid, block, 0, st, p);
   } else {
     if (out32)
-      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false, true>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_quad<C, false, true>), grid, block, 0, st, p);
     else
-      hipLaunchKernelGGL((gemm_quad<C, Cfg3<BL>, false, false>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((gemm_quad<C, false, false>), grid, block, 0, st, p);
   }
   return hipGetLastError();
 }
@@ -3296,9 +3292,11 @@ inline SplitPlan plan_split(const Choice& ch, int64_t M, int64_t N, int64_t K, i
 // them in place, and a second launch recomputes them four workgroups a tile
 // (redo_list_kernel, one workgroup per CU).  In place, a flagged tile's workgroup runs a whole
 // FP32 K loop after the others have finished: on the overflow stress
-// workload (4096^3, 49 of 256 tiles flagged) it ran 222.7 us against 150.2
-// for the same shape clean.  Multi-round shapes keep the in-place redo (the
-// other workgroups go on with the next tiles meanwhile).
+// workload (4096^3, 49 of 256 tiles flagged) it ran 201 us, deferred 176, the
+// same shape clean 135.  Multi-round shapes keep the in-place redo (the
+// other workgroups go on with the next tiles meanwhile: 8192 x 4096 x 4096
+// with the same share flagged 398 us, clean 260; as four 128x128 quarters in
+// turn it ran 567).
 //
 // Only from kDeferMinStages stages: the second launch costs ~2.3 us on
 // every call (an empty list included), which stays under 3 % of a round of

@@ -1,7 +1,6 @@
-"""The persistent kernel (gemm_persistent): chunked 256x256 on shapes of
-more than one round of tiles, one workgroup per CU walking its
-tiles and issuing each next tile's first copies ahead of the previous tile's
-store.  Shapes just past one round (257..300 tiles) keep the oracle cheap;
+"""The persistent grid of 256x256 (gemm_quad) on shapes of more than one
+round of tiles: one workgroup per CU walking its tiles and issuing each next
+tile's first copies ahead of the previous tile's store.  Shapes just past one round (257..300 tiles) keep the oracle cheap;
 the full-size 8192^3 and lm_head checks in test_gpu_parity.py run on it too.
 
 Checked: values and flags against the oracle on ragged edges, both b
@@ -139,6 +138,40 @@ def test_persistent_overflow_in_later_rounds_is_redone_exactly(tile, b_t):
     assert rel(c.cpu()[~mask.cpu()], ref[~mask.cpu()]) < TOL
     # without tile flags (the C ABI's own path): the same bits
     assert torch.equal(mm_tile(ga, gb, tile, torch.float32), c)
+
+
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M, N, K", [(8192, 4096, 128), (8192, 4096, 520), (8100, 4000, 1032)])
+def test_persistent_redoes_every_tile_of_every_round(M, N, K, b_t, biased):
+    """Every chunk overflows (32 products of U(90, 140) and more), so every
+    workgroup redoes each tile it walks before it goes on to the next, whose
+    copies it has given up: the FP32-accumulating mode's bits (sums that round
+    in FP32: another order would show), with the bias, flags all set; and, without
+    flags, the same again."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = (90.0 + 50.0 * torch.rand(M, K, generator=g, device="cuda")).half()
+    b = (90.0 + 50.0 * torch.rand(K, N, generator=g, device="cuda")).half()
+    b = b.t().contiguous().t() if b_t else b
+    bias = torch.randn(N, generator=g, device="cuda").half()
+    tiles_m, tiles_n = -(-M // 256), -(-N // 256)
+    assert tiles_m * tiles_n > CUS
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(chunked, flags):
+        c = torch.full((M, N), -1.0, device="cuda", dtype=torch.float32)
+        args = (flags, M, N, K, a.stride(0), a.stride(1), b.stride(0), b.stride(1), N, 1, _lib.OUT_F32, chunked, stream)
+        if biased:
+            _lib.check(_lib.gemm_bias(a.data_ptr(), b.data_ptr(), bias.data_ptr(), c.data_ptr(), *args))
+        else:
+            _lib.check(_lib.gemm_tile(a.data_ptr(), b.data_ptr(), c.data_ptr(), *args, 0))
+        return c
+
+    assert tile_config(a, b)["tile"] == "256x256"  # (the biased call cannot force one)
+    flags = torch.zeros(tiles_m, tiles_n, device="cuda", dtype=torch.uint8)
+    want = call(0, None)
+    assert torch.equal(call(1, flags.data_ptr()), want) and bool((flags == 1).all())
+    assert torch.equal(call(1, None), want)
 
 
 WAVES = {"256x256": (4, 2)}
