@@ -36,3 +36,16 @@ def test_bias_on_the_other_tiles(M, N, K, rm, out_dtype):
     bias = rnd((N + 1,), 6).cuda()[1:]
     y = f16acc.mm(a, b, out_dtype)
     assert torch.equal(mm_bias(a, b, bias, out_dtype), y + bias)
+
+
+@pytest.mark.parametrize("M, N, K, rm", [(512, 384, 8960, True), (1024, 1000, 8192, False), (1000, 1024, 512, True),
+                                         (2048, 1536, 136, False), (2048, 1536, 3584, False)])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+def test_bias_in_the_fp32_mode(M, N, K, rm, out_dtype):
+    """chunked=False: K splits (the bias added by their finishing launch), 64x64,
+    128x96."""
+    a, w = rnd((M, K), 7).cuda(), rnd((N, K), 8).cuda()
+    b = w.t().contiguous() if rm else w.t()
+    bias = rnd((N + 1,), 9).cuda()[1:]
+    y = f16acc.mm(a, b, out_dtype, chunked=False)
+    assert torch.equal(mm_bias(a, b, bias, out_dtype, chunked=False), y + bias)
