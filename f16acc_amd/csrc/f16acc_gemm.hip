@@ -1880,6 +1880,10 @@ __device__ __forceinline__ bool quad_whole(const Params& p, int64_t m0, int64_t 
 // A wave's LDS operations run in order, so a block's reads follow its writes
 // without a wait; fp16 blocks alternate between the slice's halves, so that a
 // block is written while the one before it is read and stored.
+// Columns apart (scn != 1: a column-major c) are stored from the registers,
+// where 16 lanes hold 16 rows of a column: staged, a store's lanes would be 16
+// bytes of a row each, in as many cache lines as elements (8192 x 8192 x 1024
+// column-major: fp16 239 us staged, 171 so; fp32 283 and 169).
 // Returns whether any sum is inf or NaN (kernel.py:70-71): 0 * s summed over
 // the lane's sums is zero exactly when all are finite.  fp16 outputs are tried
 // first, two a instruction (an inf or NaN sum is one in binary16 as well; so is
@@ -1896,31 +1900,28 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
   typedef std::conditional_t<OUT32, f32x4_a4, f16x8_a2> UnitAny;
   const int r16 = lane & 15, g = lane >> 4;
   const int64_t col0 = n0 + wn * C::WTN, row0 = m0 + wm * C::WTM;
-  // whole sub-tiles: buffer stores, a lane offset per unit of a row block and
-  // a scalar offset per block, in place of a 64-bit address per store
-  const bool whole = quad_whole<C, OUT32>(p, m0, n0, wm, wn);
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      (Out*)p.c + row0 * p.scm + col0, (short)0, kOob, 0x00020000);
-  const int scm = __builtin_amdgcn_readfirstlane((int)p.scm) * (int)sizeof(Out);
   float bad = 0.f;
   f16x2 bad2 = {(f16)0.f, (f16)0.f};
+  // a block's sums, tested, with the bias
+  auto take = [&](auto row_block, auto column_block, auto tested) __attribute__((always_inline)) {
+    constexpr int i = row_block, j = column_block;
+    f32x4 v = quad_read(acc[i][j]);
+    if constexpr (tested) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bad = __builtin_fmaf(v[r], 0.f, bad);
+    }
+    if constexpr (BIASED) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = with_bias<OUT32>(v[r], bias[j / 2][4 * (j % 2) + r]);
+    }
+    return v;
+  };
   auto write = [&](auto block) __attribute__((always_inline)) {
     constexpr int i = block;
     char LDS_AS* w = slice + (OUT32 ? 0 : (i & 1) * (C::SLICE / 2));
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j) {
-      f32x4 v = quad_read(acc[i][j]);
-      if constexpr (OUT32 || BIASED) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) bad = __builtin_fmaf(v[r], 0.f, bad);
-      }
-      if constexpr (BIASED) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float b = (float)bias[j / 2][4 * (j % 2) + r];
-          v[r] = OUT32 ? v[r] + b : (float)(f16)v[r] + b;  // with_bias
-        }
-      }
+    static_for<C::FN>([&](auto column) __attribute__((always_inline)) {
+      constexpr int j = column;
+      const f32x4 v = take(block, column, std::bool_constant<OUT32 || BIASED>{});
       if constexpr (OUT32) {
         *(f32x4 LDS_AS*)(w + r16 * (U * 16) + (((4 * j + g) ^ r16) << 4)) = v;
       } else {
@@ -1934,7 +1935,7 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
         const f16x4 o = {hl[0], hl[1], hh[0], hh[1]};
         *(f16x4 LDS_AS*)(w + r16 * (U * 16) + (((2 * j + (g >> 1)) ^ r16) << 4) + (g & 1) * 8) = o;
       }
-    }
+    });
     if constexpr (!OUT32 && !BIASED) {
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad2[0] == (f16)0.f && bad2[1] == (f16)0.f)) != 0, 0)) {
         bad2 = f16x2{(f16)0.f, (f16)0.f};
@@ -1954,7 +1955,12 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
     return *(const Unit LDS_AS*)(slice + (OUT32 ? 0 : (i & 1) * (C::SLICE / 2)) + *row * (U * 16) +
                                  ((u ^ *row) << 4));
   };
-  if (whole) {
+  if (quad_whole<C, OUT32>(p, m0, n0, wm, wn)) {
+    // buffer stores, a lane offset per unit of a row block and a scalar offset
+    // per block, in place of a 64-bit address per store
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (Out*)p.c + row0 * p.scm + col0, (short)0, kOob, 0x00020000);
+    const int scm = __builtin_amdgcn_readfirstlane((int)p.scm) * (int)sizeof(Out);
     Unit v[2][NU];
     int off[NU];
     static_for<C::FM + 1>([&](auto block) __attribute__((always_inline)) {
@@ -1976,11 +1982,11 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
                                                  16 * (i - 1) * scm, 0);
       }
     });
-  } else {
-    // the edges of c, and any strides: a loop of its own, whose masks stay
-    // out of the registers of the code above
+  } else if (p.scn == 1) {
+    // the edges of c: a loop of its own, whose masks stay out of the registers
+    // of the code above
     const int64_t rows_in = p.M - row0, cols_in = p.N - col0;
-    const bool rows_ok = p.scn == 1 && ((uintptr_t)p.c & (sizeof(Out) - 1)) == 0;
+    const bool rows_ok = ((uintptr_t)p.c & (sizeof(Out) - 1)) == 0;
     static_for<C::FM>([&](auto block) __attribute__((always_inline)) {
       constexpr int i = block;
       write(block);
@@ -1989,16 +1995,32 @@ __device__ __forceinline__ bool quad_store(const Params& p, char LDS_AS* slice, 
         int row, col;
         const Unit v = unit(i, it, &row, &col);
         if (16 * i + row >= rows_in) continue;
-        Out* dst = (Out*)p.c + (row0 + 16 * i + row) * p.scm + (col0 + col) * p.scn;
+        Out* dst = (Out*)p.c + (row0 + 16 * i + row) * p.scm + col0 + col;
         if (rows_ok && col + EL <= cols_in) {
           *(UnitAny*)dst = v;
         } else {
 #pragma unroll
           for (int e = 0; e < EL; ++e)
-            if (col + e < cols_in) dst[e * p.scn] = v[e];
+            if (col + e < cols_in) dst[e] = v[e];
         }
       }
       __builtin_amdgcn_wave_barrier();
+    });
+  } else {
+    static_for<C::FM>([&](auto block) __attribute__((always_inline)) {
+      constexpr int i = block;
+      const int64_t row = row0 + 16 * i + r16;
+      static_for<C::FN>([&](auto column) __attribute__((always_inline)) {
+        constexpr int j = column;
+        const f32x4 v = take(block, column, std::true_type{});
+        const int64_t col = col0 + 16 * j + 4 * g;
+        Out* dst = (Out*)p.c + row * p.scm + col * p.scn;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (row < p.M && col + r < p.N) dst[r * p.scn] = (Out)v[r];
+      });
+      float& tested = bad;
+      asm volatile("" : "+v"(tested));
     });
   }
   return !(bad == 0.f);

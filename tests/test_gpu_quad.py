@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from f16acc_amd import _lib
-from f16acc_amd.kernel import mm_flags, mm_tile
+from f16acc_amd.kernel import mm_flags, mm_tile, tile_config
 from oracle import chunk32
 
 pytestmark = pytest.mark.gpu
@@ -62,6 +62,41 @@ def test_quad_strided_output(out_dtype, esize):
         assert torch.equal(view, want), (scm, scn)
         view.fill_(7.0)
         assert bool((buf == 7.0).all()), (scm, scn)
+
+
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("M, N", [(4096, 4096), (4090, 8187)])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+def test_quad_column_major_output(out_dtype, M, N, biased):
+    """Columns apart are stored from the registers: one round and several, a
+    bias, an overflowing element (flagged, redone, stored again), edges; and the
+    FP32 mode."""
+    K = 520
+    a, b = rnd((M, K), 23), rnd((N, K), 24)
+    a[M - 3, 64:96] = 100.0
+    b[N - 5, 64:96] = 100.0
+    a, b = a.cuda(), b.cuda().t()
+    assert tile_config(a, b)["tile"] == TILE
+    bias = rnd((N,), 25).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    out = _lib.OUT_F32 if out_dtype == torch.float32 else _lib.OUT_F16
+
+    def call(c, scm, scn, chunked):
+        flags = torch.zeros(-(-M // 256), -(-N // 256), device="cuda", dtype=torch.uint8)
+        args = (flags.data_ptr(), M, N, K, K, 1, 1, K, scm, scn, out, chunked, stream)
+        if biased:
+            _lib.check(_lib.gemm_bias(a.data_ptr(), b.data_ptr(), bias.data_ptr(), c.data_ptr(), *args))
+        else:
+            _lib.check(_lib.gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), *args))
+        return flags
+
+    for chunked in (1, 0):
+        want = torch.empty(M, N, device="cuda", dtype=out_dtype)
+        flags = call(want, N, 1, chunked)
+        assert int(flags.sum()) == chunked and int(flags[-1, -1]) == chunked
+        buf = torch.full((N * M + 8,), 7.0, device="cuda", dtype=out_dtype)
+        assert torch.equal(call(buf, 1, M, chunked), flags)
+        assert torch.equal(buf[:N * M].view(N, M).t(), want) and bool((buf[N * M:] == 7.0).all())
 
 
 @pytest.mark.parametrize("b_t", [True, False])
