@@ -94,8 +94,8 @@ constexpr bool kRedo = !F16ACC_NO_REDO;
 constexpr bool kSplitRedo = F16ACC_SPLIT_REDO && kRedo;
 
 // F16ACC_NO_PERSISTENT=1 runs multi-round shapes on the one-tile-per-
-// workgroup grid instead of gemm_quad's walk over them; only
-// the benchmark's A/B of the two builds loads it (same bits either way).
+// workgroup grid instead of a walk over them (gemm_quad,
+// gemm_persistent); only the benchmark's A/B of the two builds loads it (same bits either way).
 #ifndef F16ACC_NO_PERSISTENT
 #define F16ACC_NO_PERSISTENT 0
 #endif
@@ -837,9 +837,9 @@ __device__ __forceinline__ void group_reduce(char LDS_AS* smem, int g, int ltid,
 // The fast path's K loop over [kbeg, kend) for this thread's K group, then
 // the group reduction: group 0 ends with the tile's sum.
 
-// Chunked K loop of the 64x144-per-wave tile (256x288), with the
-// stage barrier moved from a stage's start to before its last column: a
-// two-stage ring, where a wave that reaches the barrier has read every
+// Chunked K loop of the 64x128- and 64x144-per-wave tiles (256x256 at a short
+// K, 256x288), with the stage barrier moved from a stage's start to before its
+// last column: a two-stage ring, where a wave that reaches the barrier has read every
 // fragment of stage s (its last b column is in registers) and has its own
 // copies of stage s + 1 landed, so after the barrier it multiplies stage
 // s's last column while it reads stage s + 1's b(0) and, block by block
@@ -853,18 +853,30 @@ __device__ __forceinline__ void group_reduce(char LDS_AS* smem, int g, int ltid,
 // Same operations in the same order as k_loop_fast (same bits); measured
 // 0.9-1.4 % faster on Qwen2.5-1.5B gate/up.  (FP32 accumulation keeps k_loop_fast: there this form ran 2-6 %
 // slower.)
-template <class C>
+//
+// entry (gemm_persistent's tile chaining): kIssueFirst, the loop issues stage
+// 0's copies itself; kFirstThenStores, they were issued before exactly STORES
+// more vector memory instructions of this wave (a tile's output stores), so
+// waiting until STORES remain outstanding has them landed (vmcnt counts in
+// issue order) while the stores drain; kFirstIssued, issued before an unknown
+// number of others: wait for everything.
+enum Entry { kIssueFirst = 0, kFirstThenStores = 1, kFirstIssued = 2 };
+
+template <class C, int STORES = 0>
 __device__ __forceinline__ void k_loop_cross(const Params& p, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
                                              char LDS_AS* smem, FastLoader<C>& ld, int wave, int wm, int wn, int lane,
-                                             f32x4 (&acc)[C::FM][C::FN]) {
+                                             f32x4 (&acc)[C::FM][C::FN], int entry = kIssueFirst) {
   constexpr int T = C::FM * C::FN, kUnits = C::LA + C::LB;
   static_assert(kUnits <= T - C::FM, "copies must go out before the last column");
   static_assert(C::NS == 2 && C::KG == 1 && C::FM > 1, "two-stage ring, one K group");
   const int64_t nsteps = kend > kbeg ? (kend - kbeg + kStageK - 1) / kStageK : 0;
-  if (nsteps <= 0) return;
+  if (nsteps <= 0) return;  // (gemm_persistent runs at K > 0)
   const int r16 = lane & 15, g = lane >> 4;
-  ld.issue(p, m0, n0, kbeg, kend, smem, wave);
-  wait_vm0();
+  if (entry == kIssueFirst) ld.issue(p, m0, n0, kbeg, kend, smem, wave);
+  if (entry == kFirstThenStores)
+    wait_vm<STORES>();
+  else
+    wait_vm0();
   __syncthreads();
   f16x8 af[C::FM][2], bc[2], bn[2];
   bc[0] = read_b<C>(smem + C::A_STAGE, wn, 0, 0, lane);
@@ -2501,6 +2513,120 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
   }
 }
 
+// ---------------------------------------------------------------------------
+// 256x256 on eight waves (Cfg0: pairs of chunks, 64x128 a wave), chunked, on
+// shapes of more than one round of tiles at the short K where it beats
+// gemm_quad (quad_256).  One workgroup per CU walks the tiles blockIdx.x,
+// blockIdx.x + G, ... (G = gridDim.x, a multiple of the 8 XCDs) in the block ->
+// tile order of a whole grid.  At a tile's end the workgroup flags it (one
+// barrier), redoes it in FP32 if flagged (kernel.py:70-81), and then issues
+// the next tile's first-stage copies into ring slot 0 before staging and
+// storing this tile through the rest of the LDS: the next tile's first wait
+// covers those copies only (exactly STORES stores follow them in a wave with
+// a whole sub-tile), so the stores drain while the next tile's first stage is
+// multiplied.  8192 x 8192, fp16 out: K = 64 39.7 us against 42.4 on
+// gemm_quad and 42.3 on a grid of one tile per workgroup, K = 192 57 against
+// 60 and 59.
+// ---------------------------------------------------------------------------
+template <class C, bool OUT32>
+struct PersistentStore {
+  // the staging area: ring slot 1 onwards
+  static constexpr int AREA = C::RINGS - C::STAGE;
+  static constexpr int NW = C::WAVES_M * C::WAVES_N;
+  // fp16: the fewest column passes whose slices fit the area
+  static constexpr int P16 = passes(C::FN, (NW * C::WTM * C::WTN * 2 + AREA - 1) / AREA);
+  static constexpr int STORES16 = P16 * (C::WTM * (2 * C::FN / P16) / 64);
+  // fp32 (store_tile_staged32 with SMEM = AREA)
+  static constexpr int P32 = passes(C::FN, (NW * C::WTM * C::WTN * 4 + AREA - 1) / AREA);
+  static constexpr int STORES32 = P32 * (C::WTM * (C::WTN / P32 / 4) / 64);
+  static constexpr int STORES = OUT32 ? STORES32 : STORES16;
+  static_assert(STORES <= 63, "the stores must fit vmcnt");
+  static_assert(NW * C::WTM * (2 * C::WTN / P16) <= AREA, "fp16 staging slices must fit");
+  __device__ static __forceinline__ void store(const Params& p, char LDS_AS* area, int64_t m0, int64_t n0, int wave,
+                                               int wm, int wn, int lane, const f32x4 (&acc)[C::FM][C::FN],
+                                               const Bias<C>& bias) {
+    if constexpr (OUT32)
+      store_tile_staged32<C, AREA>(p, m0, n0, wm, wn, lane, wave, area, acc, bias);
+    else
+      store_tile_staged<C, P16>(p, m0, n0, wm, wn, lane, wave, area, acc, bias);
+  }
+};
+
+template <class C, bool OUT32>
+__global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(C::WPE))) void gemm_persistent(Params p) {
+  static_assert(C::KG == 1 && C::NS == 2 && C::FM * C::FN >= 32, "k_loop_cross's tiles");
+  using PS = PersistentStore<C, OUT32>;
+  __shared__ __attribute__((aligned(1024))) char smem_raw[C::RINGS];
+  __shared__ int flag_word[2];  // tile i raises word i & 1; the other is cleared meanwhile
+  char LDS_AS* smem = (char LDS_AS*)smem_raw;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
+  const uint32_t tiles_m = (uint32_t)p.tiles_m, tiles_n = (uint32_t)p.tiles_n, tiles = tiles_m * tiles_n;
+  uint32_t t = blockIdx.x;
+  if (t >= tiles) return;
+  if (tid == 0) flag_word[0] = flag_word[1] = 0;  // ordered before any raise by the K loop's barriers
+  int64_t tm, tn;
+  group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &tm, &tn);
+  int entry = kIssueFirst;
+  for (int it = 0;; ++it) {
+    const int64_t m0 = tm * C::BM, n0 = tn * C::BN;
+    // opaque once per tile: lane-dependent addresses are computed inside the
+    // tile loop instead of kept (and spilled) across the K loop
+    int tid_t = tid;
+    asm volatile("" : "+v"(tid_t));
+    const int lane_t = tid_t & 63;
+    FastLoader<C> ld;
+    ld.init(p, m0, n0, tid_t);
+    f32x4 acc[C::FM][C::FN];
+#pragma unroll
+    for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    k_loop_cross<C, PS::STORES>(p, m0, n0, 0, p.K, smem, ld, wave, wm, wn, lane_t, acc, entry);
+    if constexpr (kRedo) {
+      // tile flag: any element of the FP32 sum inf or NaN (kernel.py:70-71)
+      int LDS_AS* word = (int LDS_AS*)&flag_word[it & 1];
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::FN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) bad |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+      if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane_t == 0) *word = 1;
+      __syncthreads();
+      const int flag = *word;
+      // the other word's last reads were a tile ago; its next raise comes
+      // after the next tile's barriers
+      if (tid_t == 0) flag_word[(it + 1) & 1] = 0;
+      if (p.flags && tid_t == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
+      if (__builtin_expect(flag, 0)) {
+        // redo the whole tile, all of K, with FP32 accumulation (kernel.py:75-81)
+#pragma unroll
+        for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+          for (int j = 0; j < C::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        k_loop_fast<C, false>(p, m0, n0, 0, p.K, smem, ld, wave, wm, wn, lane_t, acc);
+      }
+    }
+    t += gridDim.x;  // (no wrap: both are below 2^31)
+    const bool next = t < tiles;
+    if (next) {
+      group_m<uint32_t>(xcd_order<uint32_t>(t, tiles), tiles_m, tiles_n, &tm, &tn);
+      FastLoader<C> nld;
+      nld.init(p, tm * C::BM, tn * C::BN, tid_t);
+      nld.issue(p, tm * C::BM, tn * C::BN, 0, p.K, smem, wave);  // into slot 0, free since the last barrier
+    }
+    PS::store(p, smem + C::STAGE, m0, n0, wave, wm, wn, lane_t, acc, Bias<C>(p, n0, wn, lane_t));
+    if (!next) return;
+    const int64_t rows_in = p.M - (m0 + wm * C::WTM), cols_in = p.N - (n0 + wn * C::WTN);
+    const bool whole = p.vec_store && rows_in >= C::WTM && cols_in >= C::WTN && !p.bias && !p.flags;
+    entry = whole ? kFirstThenStores : kFirstIssued;
+    __syncthreads();  // every wave's staging reads done: the next stage's copies may overwrite slot 1
+  }
+}
+
 // The redo launch of the deferred list (RedoList): the tiles a chunked
 // 256x256 launch flagged, each recomputed whole with FP32 accumulation
 // (kernel.py:75-81) as its four 128x128 quarters by four workgroups of C
@@ -2734,7 +2860,7 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 // ---------------------------------------------------------------------------
 // Tile configurations (ids are the F16ACC_TILE_* values of include/f16acc.h).
 //   id  tile     waves  wave tile  LDS ring      workgroups per CU (LDS)
-//   0   256x256  4      128x128    160 KiB       1   (gemm_quad)
+//   0   256x256  4      128x128    160 KiB       1   (gemm_quad; at a short K, 8 waves of 64x128, 2 x 64 KiB)
 //   1   256x128  8      64x64      3 x 48 KiB    1
 //   2   128x256  8      64x64      3 x 48 KiB    1
 //   3   128x128  4      64x64      2 x 32 KiB    2
@@ -2744,6 +2870,7 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 //                                                    groups of 2 x 2 waves of 64x48)
 //   7   64x32    4 x 2  32x32      2 x (2 + 3) x 12 KiB  1   (four K groups, split phases)
 //   8   256x288  8      64x144     2 x 68 KiB    1   (K-contiguous b)
+template <int BL> using Cfg0 = Cfg<256, 256, 4, 2, 2, BL>;
 template <int BL> using Cfg1 = Cfg<256, 128, 4, 2, 3, BL>;
 template <int BL> using Cfg2 = Cfg<128, 256, 2, 4, 3, BL>;
 template <int BL> using Cfg3 = Cfg<128, 128, 2, 2, 2, BL>;
@@ -3212,8 +3339,39 @@ hipError_t launch_fast(const Params& p, int blayout, int out32, int chunked, hip
                         : launch_cfg<CF<kNC>, LD>(p, out32, chunked, st);
 }
 
-// 256x256: one workgroup per tile, or on shapes of more than one round one
-// per CU, each walking its tiles.
+// 256x256: gemm_quad, or the eight-wave kernel (Cfg0).
+//
+// Chunked: a quad costs its 128 K even where its second half lies past K, so at
+// a short K whose last quad is at most half full the pair form on eight waves is
+// the faster one.  fp16 out, 4096 x 4096: K = 64 13.0 us against 14.1, 192 16.3
+// against 17.0, 320 20.2 against 20.9, 448 24.2 against 24.4; 8192 x 8192 (four
+// rounds): K = 64 39.7 against 42.4, 192 57 against 60, 320 73 against 81.  (fp32
+// out in one round 18.2 against 17.4 at K = 64: taken all the same, since c must
+// not decide how a and b are summed.)  Whole quads win from K = 128 (14.5
+// against 14.3), and so do rows that are not 16-byte aligned over several rounds
+// (N % 8; 8191 x 8187 x 64 fp32 65 against 74), where the pair form would walk
+// its tiles behind unaligned stores.
+//
+// FP32 accumulation (both kernels sum every element's chunks in order: the same
+// bits, so c may decide): no sparse MFMAs to save, and one wave per SIMD fills and
+// drains its tile alone.  Eight waves against quads, fp16 out: 4096 x 4096 K =
+// 256 14.5 us against 16.6, 1024 31.8 against 32.9, 1536 44.2 against 44.8;
+// 8192 x 8192 K = 256 51.4 against 51.8, 512 76.2 against 73.5; unaligned rows, 4093 x
+// 4089 K = 1024 33.5 against 35.5, 2560 71.6 against 71.7.  fp32 out: 4096 x 4096 K =
+// 512 25.1 against 25.0; 8192 x 8192 K = 256 65 against 76, 1024 141 against 146,
+// 2560 314 against 311; unaligned, 4093 x 4089 K = 1024 39.7 against 38.7, 8191 x
+// 8187 K = 64 65 against 62.
+inline bool quad_256(const Params& p, int out32, int chunked, int cus) {
+  const int64_t tiles = p.tiles_m * p.tiles_n;
+  if (chunked) return p.K > 320 || cdiv(p.K, kStageK) % 2 == 0 || (tiles > cus && p.N % 8 != 0);
+  if (p.K >= 2560) return true;
+  const bool many = tiles >= 3 * (int64_t)cus;
+  if (out32) return p.vec_store ? !many && p.K >= 1024 : many || p.K >= 1024;
+  return p.vec_store && p.K >= (many ? 512 : 1536);
+}
+
+// One workgroup per tile, or on shapes of more than one round one per CU, each
+// walking its tiles.
 template <int BL>
 hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStream_t st) {
   using C = QuadCfg<256, 256, BL>;
@@ -3231,6 +3389,21 @@ hipError_t launch_quad(const Params& p, int out32, int chunked, int cus, hipStre
     else
       hipLaunchKernelGGL((gemm_quad<C, false, false>), grid, block, 0, st, p);
   }
+  return hipGetLastError();
+}
+
+// The eight-wave 256x256: chunked shapes of more than one round walk their
+// tiles where rows of c are 16-byte aligned.
+template <int BL>
+hipError_t launch_256(const Params& p, int out32, int chunked, int cus, hipStream_t st) {
+  using C = Cfg0<BL>;
+  if (!kPersistent || !chunked || p.K == 0 || !p.vec_store || p.tiles_m * p.tiles_n <= cus || cus % kNumXcd != 0 ||
+      p.defer_redo)
+    return launch_cfg<C, kDma>(p, out32, chunked, st);
+  if (out32)
+    hipLaunchKernelGGL((gemm_persistent<C, true>), dim3((unsigned)cus), dim3(C::T), 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_persistent<C, false>), dim3((unsigned)cus), dim3(C::T), 0, st, p);
   return hipGetLastError();
 }
 
@@ -3499,6 +3672,9 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
                                           : (int)launch_fast<Cfg3, kReg>(q, ch.blayout, out32, chunked, st);
     switch (ch.tile) {
       case 0:
+        if (!quad_256(q, out32, chunked, cu_count()))
+          return ch.blayout == kKC ? (int)launch_256<kKC>(q, out32, chunked, cu_count(), st)
+                                   : (int)launch_256<kNC>(q, out32, chunked, cu_count(), st);
         return ch.blayout == kKC ? (int)launch_quad<kKC>(q, out32, chunked, cu_count(), st)
                                  : (int)launch_quad<kNC>(q, out32, chunked, cu_count(), st);
       case 1: return (int)launch_fast<Cfg1>(q, ch.blayout, out32, chunked, st);

@@ -142,7 +142,8 @@ def test_persistent_overflow_in_later_rounds_is_redone_exactly(tile, b_t):
 
 @pytest.mark.parametrize("biased", [False, True])
 @pytest.mark.parametrize("b_t", [False, True])
-@pytest.mark.parametrize("M, N, K", [(8192, 4096, 128), (8192, 4096, 520), (8100, 4000, 1032)])
+@pytest.mark.parametrize("M, N, K", [(8192, 4096, 64), (8192, 4096, 128), (8100, 4000, 320), (8192, 4096, 520),
+                                     (8100, 4000, 1032)])
 def test_persistent_redoes_every_tile_of_every_round(M, N, K, b_t, biased):
     """Every chunk overflows (32 products of U(90, 140) and more), so every
     workgroup redoes each tile it walks before it goes on to the next, whose
