@@ -3518,16 +3518,21 @@ inline bool deferred_redo(const Choice& ch, int64_t M, int64_t N, int64_t K, int
 inline bool wave_128x96(const Params& p) { return p.K >= 3 * 4 * 4 * kChunk; }
 
 // 64x64 tiles of at most one per CU, chunked: four waves, each a quarter of K
-// (gemm_wave), from a quad a wave on.  One workgroup of the ordinary kernel
-// alone on its CU waits out a copy's latency every 64 K: 1024 x 1024 x 1024 fp32
-// out 10.9 -> 8.75 us a call.  Two or more workgroups on a CU hide each other's
+// (gemm_wave), from K = 704 on (a row-major b: past 768, six quads).  One
+// workgroup of the ordinary kernel alone on its CU waits out a copy's latency
+// every 64 K; the four waves wait for one ring's fill and add four sums, and the
+// longest of them sets the time, so that a fifth quad costs as much as a second
+// each.  1024 x 1024, us a call, ordinary against quarters: w.t() K = 512 6.0 and
+// 6.1, 576 6.2 and 6.9, 648 6.9 and 7.3, 704 6.9 and 6.9, 768 7.1 and 6.9, 1024
+// 8.3 and 7.2; row-major b 512 6.0 and 6.3, 640 6.6 and 7.2, 768 7.1 and 7.2, 776
+// 7.6 and 7.3, 1024 8.4 and 7.5 (1000 x 1000: 776 8.0 and 8.1, 1024 8.8 and 8.5).  Two or more workgroups on a CU hide each other's
 // waits and keep the ordinary kernel (2048 x 1024 x 1024: 10.3 us against 13.3
 // in K groups; 1536 x 1024 x 2048: 17.4 against 19.7), as do the second launch
 // of a cut (one grid's summation order) and a row-major b whose 128 k-rows pass
 // 32-bit offsets.
 inline bool wave_64(const Choice& ch, const Params& p, int cus) {
   return ch.tile == F16ACC_TILE_64x64 && ch.family == F16ACC_FAMILY_FAST && p.tiles_m * p.tiles_n <= cus &&
-         p.K >= 4 * 4 * kChunk &&
+         (ch.blayout == kKC ? p.K >= 704 : p.K > 768) &&
          (ch.blayout == kKC || (int64_t)4 * kChunk * p.sbk * 2 + 2 * 64 < kOob);
 }
 

@@ -1,7 +1,7 @@
 """The K-quarter kernel (each wave a quarter of K: 128x96 from K = 1536, 64x64
-with at most one tile per CU) where its schedule can go wrong: K around whole
-quads and around the rules' lines, ragged tiles, both output types, an overflow
-in any quarter."""
+with at most one tile per CU from K = 704, 776 with a row-major b) where its
+schedule can go wrong: K around whole quads and around the rules' lines, ragged
+tiles, both output types, an overflow in any quarter."""
 
 import pytest
 import torch
@@ -42,7 +42,8 @@ def picks_64(a, b):
 
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("M, N, K", [(1024, 1024, 512), (1024, 1024, 1024), (1000, 1016, 520), (961, 1024, 648),
-                                     (1024, 968, 1160), (1023, 1000, 1544)])
+                                     (1024, 968, 1160), (1023, 1000, 1544), (1024, 1024, 696),
+                                     (1024, 1024, 704), (1000, 1016, 768), (1024, 1000, 776)])
 def test_64x64_in_k_quarters_against_one_wave_group(M, N, K, b_t):
     """At most one 64x64 tile per CU runs in wave K groups; 128x128 sums K in
     order.  The same rounded chunks in another FP32 order (sums
@@ -60,13 +61,13 @@ def test_64x64_in_k_quarters_against_one_wave_group(M, N, K, b_t):
 
 @pytest.mark.parametrize("b_t", [False, True])
 @pytest.mark.parametrize("quarter", range(4))
-def test_64x64_redoes_an_overflow_in_any_quarter(quarter, b_t):
+@pytest.mark.parametrize("K", [512, 1024])  # one wave group, four
+def test_64x64_redoes_an_overflow_in_any_quarter(K, quarter, b_t):
     """The overflow closed form (chunk sums past 65504 that cancel: exactly 100
     in FP32) in one wave's K range, the other ranges zero there."""
     M = N = 1024
-    K = 512
     a, b = rnd((M, K), 33), rnd((K, N), 34)
-    r0, c0, k0 = 64 * 5 + 20, 64 * 11 + 40, 128 * quarter
+    r0, c0, k0 = 64 * 5 + 20, 64 * 11 + 40, K // 4 * quarter
     a[r0:r0 + 10, :] = 100.0
     b[:, c0:c0 + 10] = 0.0
     for q, v in enumerate((30.0, -30.0, 30.0, -30.0)):
