@@ -2441,8 +2441,9 @@ __device__ __forceinline__ void wave_reduce(char LDS_AS* smem, int wave, int lan
     }
 }
 
-// R: the tile's configuration whose K loop redoes an overflowing tile, so that
-// it equals the FP32 mode of that tile (WaveCfg itself where that runs here).
+// R: a configuration of the tile whose FP32 K loop redoes it where it
+// overflows, with the sums of the one the FP32 mode runs (WaveCfg itself where
+// that runs here).
 template <class C, class R, bool CHUNKED, bool OUT32>
 __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_wave(Params p) {
   __shared__ __attribute__((aligned(1024))) char smem_raw[C::LDS];
@@ -2498,16 +2499,18 @@ __global__ __launch_bounds__(C::T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
         store_any<S, OUT32, C::LDS>(p, ring, m0, n0, 0, wave, 0, lane, sum, bias);
       } else {
         static_assert(R::T == C::T && R::BM == C::BM && R::BN == C::BN && R::RINGS <= C::LDS, "the same tile");
-        const int wm = wave / R::WAVES_N, wn = wave % R::WAVES_N;
+        const int g = wave / R::NWG, lw = wave % R::NWG, ltid = tid - g * R::TG;
+        const int wm = lw / R::WAVES_N, wn = lw % R::WAVES_N;
         f32x4 all[R::FM][R::FN];
 #pragma unroll
         for (int i = 0; i < R::FM; ++i)
 #pragma unroll
           for (int j = 0; j < R::FN; ++j) all[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         FastLoader<R> fl;
-        fl.init(p, m0, n0, tid);
-        k_loop_fast<R, false>(p, m0, n0, 0, p.K, smem, fl, wave, wm, wn, lane, all);
-        store_any<R, OUT32, C::LDS>(p, smem, m0, n0, wave, wm, wn, lane, all, Bias<R>(p, n0, wn, lane));
+        fl.init(p, m0, n0, ltid);
+        k_groups_fast<R, false>(p, m0, n0, 0, p.K, smem, fl, g, ltid, lw, wm, wn, lane, all);
+        if (g == 0)
+          store_any<R, OUT32, C::LDS>(p, smem, m0, n0, lw, wm, wn, lane, all, Bias<R>(p, n0, wn, lane));
       }
     }
   }
@@ -2883,6 +2886,9 @@ using CfgG = Cfg<128, 128, 2, 2, 2, kKC>;
 // ones on three (140 KiB and 120 KiB of LDS).  Measured against one phase:
 // Qwen2.5-1.5B k/v 7.67 -> 7.35 us (per call, same bits).
 using Cfg6 = Cfg<128, 96, 2, 2, 2, kKC, 2, 2, 3>;
+// Its two K groups on four waves, for the redo of a tile gemm_wave ran (the
+// FP32 mode's bits below K = 4096): two waves of 64x96 a group.
+using Cfg6Redo = Cfg<128, 96, 2, 1, 2, kKC, 2, 2>;
 using Cfg7 = Cfg<64, 32, 2, 1, 2, kKC, 2, 4, 3>;
 // 256x288: 256x256 widened by a ninth column block per wave (64x144), so
 // that 2048 x 8960 is one round of 256 tiles (8 x 32) instead of 280 256x256
@@ -3510,12 +3516,23 @@ inline bool deferred_redo(const Choice& ch, int64_t M, int64_t N, int64_t K, int
   return tiles <= cus && tiles <= kRedoMax;
 }
 
-// 128x96 in wave K groups (gemm_wave) from three quads a wave on: below, filling
-// four rings and adding four sums cost more than the loop saves.
-// Per call against two K groups, 2048 x 1536: K = 512 10.5 us against 9.6, 768
-// 12.7 against 11.4, 1280 15.9 against 15.2, 1536 17.5 against 17.7, 2048 20.7
-// against 22.1 (1536 x 1536 and 1407 x 2005 cross at the same K).
-inline bool wave_128x96(const Params& p) { return p.K >= 3 * 4 * 4 * kChunk; }
+// 128x96 in wave K groups (gemm_wave), or in two K groups of four waves (Cfg6).
+// The waves wait for four rings' fill and add four sums, and the longest of them
+// sets the time: a quad left over costs as much as four.  Chunked, from twelve
+// quads, but not at thirteen; FP32 mode, where the loop saves no MFMAs, from 32,
+// and whole quads a wave from 24.  us a call, two groups against wave groups, 2048 x
+// 1536: chunked K = 1280 15.2 and 15.9, 1536 17.6 and 17.6, 1664 18.9 and 19.7, 1792
+// 20.2 and 20.0, 2048 21.9 and 20.5, 2560 25.9 and 24.0; FP32 mode 1536 14.5 and
+// 15.7, 2560 21.5 and 21.6, 3072 23.5 and 23.2, 3200 24.1 and 24.6, 3584 26.6 and
+// 25.6, 3840 28.2 and 28.2, 4096 30.0 and 28.1 (1536 x 1536 and 1407 x 2005 cross
+// at the same K).  Where only the chunked mode runs wave groups, an overflowing
+// tile is redone in two groups (Cfg6Redo) to keep the FP32 mode's bits, ~3 us slower
+// than in wave groups (2048 x 1536 x 1536, 22 % of the blocks hot: 32.0 against
+// 28.7).
+inline bool wave_128x96(int64_t K, int chunked) {
+  const int64_t quads = cdiv(K, 4 * kChunk);
+  return quads >= (chunked ? 14 : 32) || (quads >= (chunked ? 12 : 24) && quads % 4 == 0);
+}
 
 // 64x64 tiles of at most one per CU, chunked: four waves, each a quarter of K
 // (gemm_wave), from K = 704 on (a row-major b: past 768, six quads).  One
@@ -3691,8 +3708,9 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
                                    : (int)launch_wave<WaveCfg<4, 4, kNC>, Cfg5<kNC>>(q, out32, chunked, st);
         return (int)launch_fast<Cfg5>(q, ch.blayout, out32, chunked, st);
       case 6:
-        return wave_128x96(q) ? (int)launch_wave<WaveCfg<8, 6, kKC>, WaveCfg<8, 6, kKC>>(q, out32, chunked, st)
-                              : (int)launch_cfg<Cfg6, kDma>(q, out32, chunked, st);
+        if (!wave_128x96(K, chunked)) return (int)launch_cfg<Cfg6, kDma>(q, out32, chunked, st);
+        return wave_128x96(K, 0) ? (int)launch_wave<WaveCfg<8, 6, kKC>, WaveCfg<8, 6, kKC>>(q, out32, chunked, st)
+                                 : (int)launch_wave<WaveCfg<8, 6, kKC>, Cfg6Redo>(q, out32, chunked, st);
       case 7: return (int)launch_cfg<Cfg7, kDma>(q, out32, chunked, st);
       case 8: return (int)launch_cfg<Cfg8, kDma>(q, out32, chunked, st);
       default: return (int)launch_cfg<CfgG, kGather>(q, out32, chunked, st);

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import f16acc_amd as f16acc
-from f16acc_amd.kernel import mm_flags, mm_tile, tile_config
+from f16acc_amd.kernel import mm_bias, mm_flags, mm_tile, tile_config
 from oracle import chunk32
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +100,31 @@ def test_128x96_redoes_an_overflow_in_any_quarter(quarter):
     assert bool((c[r0:r0 + 10, c0:c0 + 10] == 100.0).all())
     full = mm_tile(ga, gb, TILE, torch.float32, chunked=False)
     assert torch.equal(c[128:256, 96:192], full[128:256, 96:192])
+
+
+@pytest.mark.parametrize("K", [1280, 1536, 1600, 1672, 1792, 2056, 2560, 3072, 3200, 3584, 4096, 4104])
+def test_128x96_redone_tiles_are_the_fp32_modes(K):
+    """Every tile overflows (products of U(90, 140), whose FP32 sums round): the
+    redo sums in the order of the kernel the FP32 mode runs at this K, two K groups
+    or four; tiles of 44 rows (none in the lower half) and 58 columns."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a = (90.0 + 50.0 * torch.rand(300, K, generator=g, device="cuda")).half()
+    b = (90.0 + 50.0 * torch.rand(250, K, generator=g, device="cuda")).half().t()
+    c, flags = mm_flags(a, b, torch.float32, tile=TILE)
+    assert bool((flags == 1).all())
+    assert torch.equal(c, mm_tile(a, b, TILE, torch.float32, chunked=False))
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("K", [1536, 2560, 4096])
+def test_128x96_redo_with_a_bias(K, out_dtype):
+    M, N = 2040, 1530
+    a, w, bias = rnd((M, K), 41).cuda(), rnd((N, K), 42).cuda(), rnd((N,), 43).cuda()
+    a[256:300, 500:540] = 100.0  # tile rows 2 and 15: with these columns of b, chunks past 65504
+    a[2039, 500:540] = 100.0
+    w[:, 500:540] = w[:, 500:540].abs() * 0 + 50.0
+    assert tile_config(a, w.t())["tile"] == TILE
+    want = mm_tile(a, w.t(), TILE, out_dtype, chunked=False)[256:300]
+    c = mm_bias(a, w.t(), bias, out_dtype)
+    assert torch.equal(c[256:300], want + bias)
+    assert torch.equal(c, f16acc.mm(a, w.t(), out_dtype) + bias)
