@@ -2869,8 +2869,8 @@ __global__ __launch_bounds__(256) void pack_kernel(const f16* __restrict__ src, 
 //   3   128x128  4      64x64      2 x 32 KiB    2
 //   4   128x128  4      64x64      1 x 32 KiB    generic strided gather path
 //   5   64x64    4      32x32      2 x 16 KiB    4
-//   6   128x96   4      128x96     4 x 40 KiB    1   (gemm_wave: each wave a quarter of K; short K: two K
-//                                                    groups of 2 x 2 waves of 64x48)
+//   6   128x96   4      128x96     4 x 40 KiB    1   (gemm_wave: each wave a quarter of K; at a short K two
+//                                                    K groups of 4 waves of 64x48)
 //   7   64x32    4 x 2  32x32      2 x (2 + 3) x 12 KiB  1   (four K groups, split phases)
 //   8   256x288  8      64x144     2 x 68 KiB    1   (K-contiguous b)
 template <int BL> using Cfg0 = Cfg<256, 256, 4, 2, 2, BL>;
@@ -2895,6 +2895,7 @@ using Cfg7 = Cfg<64, 32, 2, 1, 2, kKC, 2, 4, 3>;
 // tiles; K-contiguous b only (288 columns are 36 units of a k-row).
 using Cfg8 = Cfg<256, 288, 4, 2, 2, kKC>;
 
+// threads: of a tile's chunked kernel; 256x256 and 128x96 have two (chunked_threads)
 struct TileInfo {
   int bm, bn, threads, per_cu;
 };
@@ -3367,9 +3368,12 @@ hipError_t launch_fast(const Params& p, int blayout, int out32, int chunked, hip
 // 512 25.1 against 25.0; 8192 x 8192 K = 256 65 against 76, 1024 141 against 146,
 // 2560 314 against 311; unaligned, 4093 x 4089 K = 1024 39.7 against 38.7, 8191 x
 // 8187 K = 64 65 against 62.
+inline bool quad_256_chunked(int64_t N, int64_t K, int64_t tiles, int cus) {
+  return K > 320 || cdiv(K, kStageK) % 2 == 0 || (tiles > cus && N % 8 != 0);
+}
 inline bool quad_256(const Params& p, int out32, int chunked, int cus) {
   const int64_t tiles = p.tiles_m * p.tiles_n;
-  if (chunked) return p.K > 320 || cdiv(p.K, kStageK) % 2 == 0 || (tiles > cus && p.N % 8 != 0);
+  if (chunked) return quad_256_chunked(p.N, p.K, tiles, cus);
   if (p.K >= 2560) return true;
   const bool many = tiles >= 3 * (int64_t)cus;
   if (out32) return p.vec_store ? !many && p.K >= 1024 : many || p.K >= 1024;
@@ -3532,6 +3536,13 @@ inline bool deferred_redo(const Choice& ch, int64_t M, int64_t N, int64_t K, int
 inline bool wave_128x96(int64_t K, int chunked) {
   const int64_t quads = cdiv(K, 4 * kChunk);
   return quads >= (chunked ? 14 : 32) || (quads >= (chunked ? 12 : 24) && quads % 4 == 0);
+}
+
+// Threads per workgroup of a chunked call on the chosen tile.
+inline int chunked_threads(const Choice& ch, int64_t N, int64_t K, int64_t tiles, int cus) {
+  if (ch.tile == F16ACC_TILE_256x256 && !quad_256_chunked(N, K, tiles, cus)) return Cfg0<kKC>::T;
+  if (ch.tile == F16ACC_TILE_128x96_K2 && !wave_128x96(K, 1)) return Cfg6::T;
+  return kTiles[ch.tile].threads;
 }
 
 // 64x64 tiles of at most one per CU, chunked: four waves, each a quarter of K
@@ -3834,7 +3845,7 @@ int f16acc_tile_config(int64_t M, int64_t N, int64_t K, int64_t sam, int64_t sak
   if (tiles_m) *tiles_m = cdiv(M, t.bm);
   if (tiles_n) *tiles_n = cdiv(N, t.bn);
   if (family) *family = ch.family;
-  if (threads) *threads = t.threads;
+  if (threads) *threads = chunked_threads(ch, N, K, cdiv(M, t.bm) * cdiv(N, t.bn), cu_count());
   return 0;
 }
 

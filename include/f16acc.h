@@ -28,14 +28,16 @@ extern "C" {
 
 /* Tile configurations of the per-shape table (f16acc_tile_config reports
  * which one a problem uses; f16acc_gemm_tile forces one). */
-#define F16ACC_TILE_256x256 0
+#define F16ACC_TILE_256x256 0 /* 4 waves of 128x128; at a short K 8 of 64x128 */
 #define F16ACC_TILE_256x128 1
 #define F16ACC_TILE_128x256 2
 #define F16ACC_TILE_128x128 3
 #define F16ACC_TILE_GENERIC 4 /* 128x128, any strides, element gather */
-#define F16ACC_TILE_64x64 5   /* small grids: 4 waves of 32x32, 4 workgroups per CU */
-#define F16ACC_TILE_128x96_K2 6 /* K groups: four waves of 128x96, each a quarter of K inside the
-                                   workgroup; K-contiguous b (else runs as 128x128) */
+#define F16ACC_TILE_64x64 5   /* small grids: 4 waves of 32x32, 4 workgroups per CU; one or
+                                 less: 4 waves, each the tile over a quarter of K */
+#define F16ACC_TILE_128x96_K2 6 /* K groups inside the workgroup: four waves of 128x96, each a
+                                   quarter of K, or at a shorter K two groups of four waves of
+                                   64x48; K-contiguous b (else runs as 128x128) */
 #define F16ACC_TILE_64x32_K4 7  /* four K groups of 2 waves of 32x32 splitting K inside the
                                    workgroup; K-contiguous b (else runs as 64x64) */
 #define F16ACC_TILE_256x288 8    /* 8 waves of 64x144; K-contiguous b (else runs as 256x256) */
@@ -177,7 +179,8 @@ int f16acc_gemm_noalloc(const void* a, const void* b, const void* bias, void* c,
  * what f16acc_gemm_tile would run with that tile (a fast tile the operands'
  * strides or alignment do not allow falls back to F16ACC_TILE_GENERIC).
  * Writes the tile id, the workgroup tile (bm x bn), the tile grid, the
- * kernel family (F16ACC_FAMILY_*) and the threads per workgroup.  Any output
+ * kernel family (F16ACC_FAMILY_*) and the threads per workgroup of a chunked
+ * call (FP32 accumulation runs some tiles with another number).  Any output
  * pointer may be NULL.
  */
 int f16acc_tile_config(int64_t M, int64_t N, int64_t K,

@@ -162,6 +162,23 @@ def test_tile_table(M, N, K, sa, sb, fam, tile):
     assert cfg["tiles_m"] == -(-M // cfg["bm"]) and cfg["tiles_n"] == -(-N // cfg["bn"])
 
 
+@pytest.mark.parametrize("M, N, K, tile, threads", [
+    # chunk quads on four waves, pairs on eight where a short K's last quad is at most half full
+    (4096, 4096, 64, "256x256", 512), (4096, 4096, 65, "256x256", 256), (4096, 4096, 128, "256x256", 256),
+    (4096, 4096, 192, "256x256", 512), (4096, 4096, 320, "256x256", 512), (4096, 4096, 321, "256x256", 256),
+    (4096, 4096, 4096, "256x256", 256), (8192, 8192, 192, "256x256", 512), (8192, 8187, 192, "256x256", 256),
+    # two K groups of four waves, four waves
+    (2048, 1536, 768, "128x96k2", 512), (2048, 1536, 1528, "128x96k2", 256), (2048, 1536, 1536, "128x96k2", 256),
+    (2048, 1536, 1408, "128x96k2", 512), (2048, 1536, 1544, "128x96k2", 512), (2048, 1536, 1664, "128x96k2", 512),
+    (2048, 1536, 1672, "128x96k2", 256), (2048, 1536, 8960, "128x96k2", 256),
+    (1024, 1024, 512, "64x64", 256), (1024, 1024, 1024, "64x64", 256), (2048, 256, 1536, "64x32k4", 512),
+])
+def test_threads_are_the_chunked_kernels(M, N, K, tile, threads):
+    ld = -(-K // 8) * 8
+    cfg = tile_config(_Fake((M, K), (ld, 1)), _Fake((K, N), (1, ld)), tile)
+    assert (cfg["tile"], cfg["threads"]) == (tile, threads)
+
+
 @pytest.mark.parametrize("tile", ["256x256", "256x128", "128x256", "128x128", "generic", "64x64", "128x96k2",
                                   "64x32k4", "256x288"])
 def test_forced_tile_resolves(tile):
