@@ -1578,11 +1578,12 @@ struct QuadCfg {
   static_assert(BL == kKC || T / UB == 8, "an NC unit's parity is bit 3 of its k-row");
 };
 
-// One copy of 16 bytes per lane to LDS, as lds_dma16, at lane offset base + step.
+// One copy of 16 bytes per lane to LDS, as lds_dma16, at lane offset base + step,
+// unsigned: kOob + step passes 2^31.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved: the asm sets it itself
 __device__ __forceinline__ void lds_dma16_step(const i32x4& srd, int lds, int base, int step) {
-  const int off = base + step;
+  const uint32_t off = (uint32_t)base + (uint32_t)step;
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
       "s_nop 0\n\t"
