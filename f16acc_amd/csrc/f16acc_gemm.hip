@@ -1475,24 +1475,6 @@ __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, 
     const int flag = tf.set_and_read(bad, lane);
     if (p.flags && tid == 0) p.flags[tm * p.tiles_n + tn] = (uint8_t)flag;
     if (__builtin_expect(!flag, 1) || (kSplitRedo && p.defer_redo)) return;
-    if (p.list) {
-      // deferred: the redo launch that follows recomputes this tile; a list
-      // that is full (or not zeroed) leaves the redo here.  The flag word
-      // carries the outcome once every wave has read the flag.
-      __syncthreads();
-      if (tid == 0) {
-        const int idx = atomicAdd(&p.list->alloc, 1);
-        const bool listed = idx >= 0 && idx < kRedoMax;
-        if (listed) {
-          store_agent(&p.list->items[idx], (int)(tm * p.tiles_n + tn));
-#pragma unroll
-          for (int j = 0; j < kLines; ++j) atomicAdd(&p.list->line[j].word, 1ull);
-        }
-        *tf.word = listed ? 2 : 1;
-      }
-      __syncthreads();
-      if (*tf.word == 2) return;
-    }
     // redo the whole tile, all of K, with FP32 accumulation (kernel.py:75-81)
 #pragma unroll
     for (int i = 0; i < C::FM; ++i)
@@ -1717,8 +1699,11 @@ __device__ __forceinline__ void chunk_quad_selector(int lane, f16x8& sel, int& i
 
 // S += the quad's four rounded chunks.  The sum stays in accumulation
 // registers ("a"), which the compiler would otherwise not mix with partials in
-// vector registers.  Four MFMAs lie between the last conversion into x and
-// this read of it, and 60 blocks between two sums of one block.
+// vector registers.  The compiler keeps no hazards for it: between the last
+// conversion into x and this read of it lie a chunk MFMA and the two conversions
+// of the next block's first chunk (an MFMA needs two wait states behind a VALU
+// write of its operand), and between two sums of one block a quad of blocks (15
+// others on 64x64, 47 on 128x96, 63 on 256x256).
 __device__ __forceinline__ void quad_sum(f32x4& s, const f16x8& sel, const f16x16& x, int idx) {
   asm("v_smfmac_f32_16x16x64_f16 %0, %1, %2, %3" : "+a"(s) : "v"(sel), "v"(x), "v"(idx));
 }
