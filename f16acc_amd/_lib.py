@@ -95,11 +95,20 @@ def check(rc):
         raise RuntimeError(strerror(rc).decode())
 
 
-def _load_host():
-    """The native call path (csrc/host.cpp)."""
-    spec = importlib.util.spec_from_file_location("f16acc_host", HOST)
-    mod = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(mod)
+def _load_host(path=HOST):
+    """The native call path (csrc/host.cpp), built for the torch that runs."""
+    spec = importlib.util.spec_from_file_location("f16acc_host", path)
+    try:
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+    except ImportError as e:
+        raise ImportError(f"{path} does not load with torch {torch.__version__} (built for another?): rebuild it") from e
+    return _for_this_torch(mod, path)
+
+
+def _for_this_torch(mod, path, version=torch.__version__):
+    if mod.torch_version != version.split("+")[0]:
+        raise ImportError(f"{path} was built for torch {mod.torch_version}, this is {version}: rebuild it")
     return mod
 
 

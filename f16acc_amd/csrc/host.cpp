@@ -25,6 +25,7 @@
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include "f16acc.h"
 
@@ -192,14 +193,32 @@ PyObject* host_setup(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+// reads(M, N, K, sam, sak, sbk, sbn, address of a, of b): read_as_they_are, for
+// its comparison with kernel.py's rules
+PyObject* host_reads(PyObject*, PyObject* args) {
+  long long M, N, K, sam, sak, sbk, sbn;
+  Py_ssize_t a, b;
+  if (!PyArg_ParseTuple(args, "LLLLLLLnn", &M, &N, &K, &sam, &sak, &sbk, &sbn, &a, &b)) return nullptr;
+  return PyBool_FromLong(read_as_they_are((const void*)a, (const void*)b, M, N, K, sam, sak, sbk, sbn));
+}
+
 PyMethodDef methods[] = {
     {"mm", (PyCFunction)(void (*)(void))host_mm, METH_FASTCALL, "mm(a, b, bias, out32, chunked) -> Tensor or None"},
     {"linear", (PyCFunction)(void (*)(void))host_linear, METH_FASTCALL,
      "linear(x, w, bias, min_rows) -> Tensor or None"},
+    {"reads", host_reads, METH_VARARGS, "reads(M, N, K, sam, sak, sbk, sbn, a, b) -> bool"},
     {"setup", host_setup, METH_VARARGS, "setup(raw_stream, pack_min_macs, 5 function addresses)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "f16acc_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_f16acc_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_f16acc_host() {
+  PyObject* m = PyModule_Create(&module);
+  // the module uses torch's C++ types, which change between versions: _lib.py checks it
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

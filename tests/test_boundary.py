@@ -429,3 +429,39 @@ def test_workspace_holds_the_redo_list_where_it_is_deferred():
         _lib.check(_lib.workspace_size(M, N, K, K, 1, sbk, sbn, 0, 0, ctypes.byref(n)))
         got = "none" if n.value == 0 else "header" if n.value == _lib.WS_HEADER else "split"
         assert got == want, (M, N, K, n.value)
+
+
+def test_native_path_is_built_for_this_torch():
+    """f16acc_host.so uses torch's C++ types: a build for another version is
+    refused at import, and so is a file that does not load."""
+    import torch
+
+    assert _lib.host.torch_version == torch.__version__.split("+")[0]
+    with pytest.raises(ImportError, match="rebuild"):
+        _lib._for_this_torch(_lib.host, "f16acc_host.so", "1.0.0+rocm1")
+    with pytest.raises(ImportError, match="rebuild"):
+        _lib._load_host(__file__.replace(".py", ".so"))
+
+
+def test_native_path_routes_as_the_general_path():
+    """csrc/host.cpp's routing rule against _pack_plan's over sizes on both sides
+    of its lines (the cost of a copy, the smallest problem worth one) and
+    strides and addresses of every kind."""
+    import random
+
+    from f16acc_amd.kernel import _pack_plan
+
+    rng = random.Random(5)
+    seen = {True: 0, False: 0}
+    sizes = [1, 2, 7, 8, 33, 64, 129, 250, 256, 300, 1000, 1001, 1024, 1536, 1537, 2048, 2049, 4096, 8191, 8961]
+    for i in range(20000):
+        M, N, K = (rng.choice(sizes) for _ in range(3))
+        pad = rng.choice([0, 0, 0, 1, 8, 16, 100])
+        sa = rng.choice([(K + pad, 1), (K + pad, 1), (1, M + pad), (0, 1), (1, 0), (2 * K, 2), (max(K // 2, 1), 1)])
+        sb = rng.choice([(N + pad, 1), (1, K + pad), (1, K + pad), (0, 1), (1, 0), (2 * N, 2), (1, max(K // 2, 1))])
+        a = _Fake((M, K), sa, 4096 + 2 * rng.choice([0, 0, 0, 1, 4, 8]))
+        b = _Fake((K, N), sb, 8192 + 2 * rng.choice([0, 0, 0, 1, 4, 8]))
+        as_they_are = _pack_plan(a, b, M, N, K)[:2] == (False, False)
+        assert _lib.host.reads(M, N, K, *sa, *sb, a.data_ptr(), b.data_ptr()) == as_they_are, (M, N, K, sa, sb)
+        seen[as_they_are] += 1
+    assert min(seen.values()) > 2000, seen
