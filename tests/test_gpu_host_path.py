@@ -52,17 +52,23 @@ def test_native_bias_and_linear_equal_general():
         for shape, N in (((128, 256), 96), ((3, 50, 64), 130), ((2, 2, 64, 200), 72), ((256, 129), 33)):
             x, w, b = rnd(*shape, seed=3), rnd(N, shape[-1], seed=4), rnd(N, seed=5)
             rows = x.numel() // shape[-1]
+            x2 = x.reshape(rows, shape[-1])
             for bias in (None, b, rnd(2 * N, seed=6)[::2]):
+                native = bias is None or bias.is_contiguous()
                 with torch.no_grad():
                     y = F.linear(x, w, bias)
-                    x2 = x.reshape(rows, shape[-1])
+                    assert (host.linear(x, w, bias, patch.MIN_ROWS) is not None) == native
                     want = kernel._mm(x2, w.t(), torch.float16, True) if bias is None else kernel._mm_bias(
                         x2, w.t(), bias, torch.float16, True)
                 assert y.shape == (*shape[:-1], N) and y.is_contiguous()
                 assert torch.equal(y.view(rows, N), want)
-            if bias is not None and bias.is_contiguous():
-                assert torch.equal(f16acc.kernel.mm_bias(x2, w.t(), b, torch.float32),
-                                   kernel._mm_bias(x2, w.t(), b, torch.float32, True))
+                for out, chunked in ((torch.float32, True), (torch.float16, False), (torch.float32, False)):
+                    c = host.mm(x2, w.t(), bias, out is torch.float32, chunked)
+                    assert (c is not None) == native
+                    if native and bias is not None:
+                        want = kernel._mm_bias(x2, w.t(), bias, out, chunked)
+                        assert c.dtype == out and torch.equal(c, want)
+                        assert torch.equal(f16acc.kernel.mm_bias(x2, w.t(), bias, out, chunked), want)
     finally:
         f16acc.disable()
 
@@ -112,12 +118,22 @@ def test_calls_left_to_the_general_path():
 def test_native_path_on_another_stream_and_in_a_graph():
     x, w = rnd(256, 512, seed=7), rnd(256, 512, seed=8)
     want = kernel._mm(x, w.t(), torch.float16, True)
+    # on s, behind work that takes milliseconds and ends by writing x: a launch on
+    # another stream would read the zeros
     s = torch.cuda.Stream()
-    s.wait_stream(torch.cuda.current_stream())
+    late = torch.zeros_like(x)
+    slow = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
     with torch.cuda.stream(s):
-        y = f16acc.mm(x, w.t())
+        for _ in range(20):
+            slow = torch.mm(slow, slow).clamp_(-1.0, 1.0)
+        late.copy_(x)
+        y = host.mm(late, w.t(), None, False, True)
+        with torch.no_grad():
+            z = host.linear(late, w, None, 128)
+    assert not s.query()
     s.synchronize()
-    assert torch.equal(y, want)
+    assert torch.equal(y, want) and torch.equal(z, want)
     g = torch.cuda.CUDAGraph()
     with torch.no_grad(), torch.cuda.graph(g):
         z = patch.linear(x, w)
