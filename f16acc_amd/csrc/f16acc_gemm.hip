@@ -3221,10 +3221,12 @@ inline int choose_tile(int64_t M, int64_t N, int64_t K, int cus, double* est = n
 // for tall problems) as whole rounds of 256x256 tiles, the rest as a second
 // GEMM with the table's own choice for that narrower shape (64x64 there:
 // four times the tiles of 128x128 fill the GPU).  Both are
-// ordinary whole-K launches on the same stream, so every output element is
-// computed exactly as in a single launch; only the tile each element's
-// overflow redo covers differs, which the reference leaves to its autotuner
-// as well.  Taken when the estimate (the table's units) gains at least 3 %;
+// ordinary launches on the same stream, and every output element sums its own
+// chunks over K in order.  In FP32 mode that gives the bits of a single launch;
+// chunked, the 256x256 part adds four chunks at a time (gemm_quad) and the second
+// launch two, so the last bit of an FP32 sum is that of the part it lies in, and
+// the tile each element's overflow redo covers differs (which the reference
+// leaves to its autotuner as well).  Taken when the estimate (the table's units) gains at least 3 %;
 // on a tie the cut whose main part fills more of its rounds wins.
 struct TailPlan {
   bool rows;   // cut along M (rows) instead of N (columns)
@@ -3542,7 +3544,7 @@ inline int chunked_threads(const Choice& ch, int64_t N, int64_t K, int64_t tiles
 // 7.6 and 7.3, 1024 8.4 and 7.5 (1000 x 1000: 776 8.0 and 8.1, 1024 8.8 and 8.5).  Two or more workgroups on a CU hide each other's
 // waits and keep the ordinary kernel (2048 x 1024 x 1024: 10.3 us against 13.3
 // in K groups; 1536 x 1024 x 2048: 17.4 against 19.7), as do the second launch
-// of a cut (one grid's summation order) and a row-major b whose 128 k-rows pass
+// of a cut (which takes no K groups) and a row-major b whose 128 k-rows pass
 // 32-bit offsets.
 inline bool wave_64(const Choice& ch, const Params& p, int cus) {
   return ch.tile == F16ACC_TILE_64x64 && ch.family == F16ACC_FAMILY_FAST && p.tiles_m * p.tiles_n <= cus &&
@@ -3639,8 +3641,8 @@ int gemm_impl(const void* a, const void* b, const void* bias, void* c, uint8_t* 
                      (char*)c + at * scn * esize, nullptr, M, N - at, K, sam, sak, sbk, sbn, scm, scn, out_dtype,
                      chunked, stream, -1, workspace, ws_bytes, strict_ws, false);
   }
-  // The second launch of a cut takes no K-group tile (kgroups false), so that
-  // every element sums its chunks in the single grid's order, bit for bit.
+  // The second launch of a cut takes no K-group tile (kgroups false): the cuts
+  // were measured without them (plan_tail), and K stays one sequence.
   const Choice ch = choose(M, N, K, sam, sak, sbk, sbn, a, b, forced_tile, kgroups);
   Params p;
   p.a = (const f16*)a;

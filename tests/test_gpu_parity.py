@@ -849,9 +849,9 @@ def test_ragged_round_tail_split_equals_single_grid(out_dtype, b_layout):
     256 CUs.  With a row-major b, mm runs columns 0..8191 as one round of
     256x256 tiles and the last 768 as a second launch (B offset by 8192
     columns); with b = w.t() it runs one round of 256 tiles of 256x288 (the
-    last column of tiles 32 wide) and no cut.  Every element is computed as
-    in the single grid mm_flags launches (bit for bit) and matches the
-    oracle."""
+    last column of tiles 32 wide) and no cut.  Every element matches the
+    oracle, and the single grid mm_flags launches (bit for bit: the FP32 sums
+    of this data come out alike in either part's order)."""
     x, w = rnd((2048, 1536), 80), rnd((8960, 1536), 81, 0.05)
     gx = x.cuda()
     gb = w.cuda().t() if b_layout == "w.t()" else w.t().contiguous().cuda()
@@ -1261,8 +1261,9 @@ def test_ragged_round_row_cut_equals_single_grid(b_layout):
     """A tall problem (8960 x 2048 x 1536: 35 x 8 tiles of 256x256 for 256
     CUs) is cut along M: rows 0..8191 as one round of 256x256 tiles, the last
     768 as a second launch (a offset by 8192 rows, c by 8192 rows).  Every
-    element is computed as in the single grid, bit for bit; the fused bias
-    is per column, so it applies unchanged to both launches."""
+    element is the single grid's, bit for bit (the FP32 sums of this data come out
+    alike in either part's order); the fused bias is per column, so it applies
+    unchanged to both launches."""
     from f16acc_amd import patch
 
     x, w, bias = rnd((8960, 1536), 110), rnd((2048, 1536), 111, 0.05), rnd((2048,), 112, 0.5)
