@@ -5,12 +5,15 @@
 // every 32-long K chunk of a dot product is summed, rounded once to binary16
 // (round to nearest even, overflow to inf) and added to an FP32 running sum;
 // an output tile whose FP32 sum ends up inf/NaN is recomputed, whole, with
-// FP32 accumulation by the same workgroup, so there is no second launch and
-// no host sync.
+// FP32 accumulation: by the same workgroup, or, where one round of 256x256
+// tiles has a long K and a workspace, by a second launch that reads a list of
+// them on the device.  There is no host sync.
 //
 // gfx950 has no FP16-accumulating MFMA, so a chunk is one
 // v_mfma_f32_16x16x32_f16 with a zero accumulator (K = 32 = one chunk), and
-// the chunk semantics are emulated per pair of chunks of a 16x16 block:
+// the chunk semantics are emulated per pair of chunks of a 16x16 block (per
+// quad, with a sparse MFMA, where a wave has the registers: gemm_quad and
+// gemm_wave below):
 //   v_cvt_pk_f16_f32  rounds the FP32 partials of two consecutive chunks of
 //                     the same element into one register (RNE, inf past 65504)
 //   selector MFMA     one more v_mfma_f32_16x16x32_f16 against a constant 0/1
@@ -1506,10 +1509,11 @@ __device__ __forceinline__ void finish_tile(const Params& p, char LDS_AS* smem, 
 // of blocks (32), two rounded quads and four partials in flight.  That also
 // reads a third less LDS per product than eight waves of 64x128.
 //
-// The bound is the chip's power: fed from registers alone, the loop's MFMAs
-// and conversions run at their full issue rate but at 1.69 GHz (3.04 us per
-// quad of a 256x256 tile, 97 us at 4096^3, where each MFMA's zero accumulator
-// and new operands toggle); the fragments, copies and barriers add the rest.
+// The bound is the one wave's issue: at 4096^3 (w.t(), 137 us under the
+// counters, 1.88 GHz) the MFMA pipe is busy 0.64 of the cycles, against 0.61 in
+// the FP32 mode and 0.71 in the library's kernel, the wave waits 0.11 in
+// s_waitcnt and barriers, and VALU instructions take 0.53 (FP32 mode 0.24), most
+// of them the conversions.
 // Measured per call against the pair form on eight waves, 4096^3 131 us
 // against 144 (w.t()), 8192^3 990 against 1078, 2048 x 8192 x 1536 55 against
 // 59.  Wider MFMAs (32x32x16, 14 % more power per product), copies spread
@@ -2958,11 +2962,18 @@ inline void canon_strides(int64_t M, int64_t N, int64_t K, int64_t* sam, int64_t
 // and the Qwen2.5-1.5B layer shapes.  Workgroups spread over the CUs, so a CU
 // ends up with ceil(tiles / CUs) tiles:
 //   estimated time = ceil(tiles / CUs) x tile area / rate.
-// 256x256 reads the least LDS per MFMA (64x128 per wave) and wins whenever
-// its tiles fill the machine; smaller tiles win on shapes with few tiles.
+// 256x256 reads the least LDS per MFMA and wins whenever its tiles fill the
+// machine; smaller tiles win on shapes with few tiles.
+// The rates are those of the kernels that sum chunk pairs, 256x256 in eight
+// waves (147 us at 4096^3) among them.  gemm_quad is faster, so against it the
+// others' true rates are lower (128x128 0.81, 256x128 0.75: 142, 174 and 189 us
+// at 4096^3 in one run), and 128x96 in K quarters is faster than its two groups,
+// which the small-grid rules were fitted to.  Of 246 checked shapes 20 run more
+// than 5 % behind the best tile, 13 of them 64x64 where 128x96 in K quarters is
+// 7-22 % faster.
 constexpr double kTileRate[4] = {1.00, 0.87, 0.87, 0.89};
 // The rate of any tile the table weighs: 256x288 (a ninth column block per
-// wave of 256x256) runs at 256x256's rate.
+// wave of the eight-wave 256x256 kernel) is priced at that kernel's rate.
 inline double tile_rate(int id) {
   return id >= F16ACC_TILE_256x256 && id <= F16ACC_TILE_128x128 ? kTileRate[id] : kTileRate[F16ACC_TILE_256x256];
 }
@@ -3077,11 +3088,13 @@ inline double rounds_256(int64_t n, int cus) {
   return rounds_of(n, cus, 256.0 * 256.0 / kTileRate[F16ACC_TILE_256x256]);
 }
 
-// 256x288 (K-contiguous b): 256x256 with a ninth column block per wave, so a
-// tile costs its area at 256x256's rate.  It wins where its tiles fill the
-// rounds better: Qwen2.5-1.5B gate/up (2048 x 8960) is 256 tiles, one round,
-// against 280 256x256 tiles (a ragged second round, or a cut with a second
-// launch for the last 768 columns).
+// 256x288 (K-contiguous b): the eight-wave 256x256 kernel with a ninth column
+// block per wave, so a tile is priced at its area at that kernel's rate (against
+// gemm_quad it is slower: 8192 x 9216 x 4096, four rounds against four and a
+// half, 666 us against 614).  It wins where its tiles fill the rounds better:
+// Qwen2.5-1.5B gate/up (2048 x 8960) is 256 tiles, one round, against 280
+// 256x256 tiles (a ragged second round, or a cut with a second launch for the
+// last 768 columns).
 inline double rounds_288(int64_t n, int cus) {
   return rounds_of(n, cus, 256.0 * 288.0 / kTileRate[F16ACC_TILE_256x256]);
 }
@@ -3089,7 +3102,8 @@ inline double rounds_288(int64_t n, int cus) {
 // K-group tiles (kc: the operands allow them, a K-contiguous b on the fast
 // path), for small grids: 128x96 where its tiles fill more
 // than half of the CUs in one round of one workgroup per CU, else 64x32 (four
-// K groups) where its tiles fit in one round at all.  Measured on MI355X:
+// K groups) where its tiles fit in one round at all.  Measured on MI355X with
+// 128x96 in two K groups (from K ~ 1536 on it runs K quarters now, wave_128x96):
 // Qwen2.5-1.5B k/v 2048x256x1536 7.96 us on 64x32 against 12.2 on 64x64
 // (kernel time; hipBLASLt 8.7); q/o 2048x1536x1536 19.5 us on 128x96 against
 // 20.4 on 64x64; down 2048x1536x8960 83.5 us on 128x96 against 87 for
