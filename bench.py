@@ -27,7 +27,7 @@ overflow flag and redo on data that never overflows; --workload persistent_ab
 times multi-round shapes on the persistent kernel against a build that runs
 them one tile per workgroup; --workload
 overflow_split_redo times the overflow stress workload against a build that
-redoes flagged tiles in a split-K pass instead of in the same workgroup;
+redoes flagged tiles in a split-K pass, and in place against the deferred list;
 --workload table_check times the per-shape table against every forced tile on
 llama-2-7B, llama-3-8B and Qwen2.5-7B layer shapes; --workload small_grid_check
 times its small-grid picks (K-group tiles, 64x64) against the other candidates,
@@ -340,7 +340,7 @@ def large_grid_check(rounds=3):
 
 
 def small_grid_check(rounds=3):
-    """The table's pick against 128x96 in two K groups, 64x32 in four, 64x64
+    """The table's pick against 128x96, 64x32 in four K groups, 64x64
     and 128x128 (each forced) on grids that leave CUs idle: x [M, K] @ w.t()
     over M 256..4096, N 256..5120, K 1024..8192 and a second grid of other
     extents, wherever the table picks a K-group tile or 64x64 (the region of
